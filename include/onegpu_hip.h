@@ -165,11 +165,9 @@ int og_int8_gemm(og_ctx *ctx, const og_int8_gemm_params *params, uint32_t batch,
 int og_int8_gemm_noalloc(og_ctx *ctx, const og_int8_gemm_params *params, uint32_t batch, og_buffer A, og_buffer B,
                          og_buffer C, og_buffer ZA, og_buffer ZB, og_buffer bias, og_buffer scale, og_buffer fbias);
 
-/* The kernel class og_int8_gemm takes for these parameters (a stable name, e.g. "mfma-i8-direct128x128x64"), the HIP
- * counterpart of Int8Gemm.Variant (Int8Gemm.cs:214-215): set by the product's rows, layout, alignment and depth. Within
- * a class the library may run another kernel where that is faster (small grids, rows that are not 16-byte aligned);
- * the name stays, and so do the result and the scratch that the class reserves. Validates nothing; writes at most len
- * bytes. */
+/* The kernel og_int8_gemm would run for these parameters (a stable name, e.g. "mfma-i8-direct256x256x64" or, a tile's rows,
+ * columns and waves, "mfma-i8-waves32x64x4"; "-splitk" where K is cut into slices), the HIP counterpart of
+ * Int8Gemm.Variant (Int8Gemm.cs:214-215). Validates nothing; writes at most len bytes. */
 int og_int8_gemm_kernel_name(const og_int8_gemm_params *params, uint32_t batch, char *buf, size_t len);
 
 /* Int8EpilogueParams, 11 words (src/RecursiveAI.OneGpu.Kernels/Shaders/Int8Epilogue.hlsl:15-28). */
@@ -348,7 +346,7 @@ int og_gather(og_ctx *ctx, uint32_t elem_bytes, const og_gather_params *params, 
 
 const char *og_last_error(og_ctx *ctx);           /* text of the last failure (thread-local when ctx is NULL) */
 const char *og_last_error_argument(og_ctx *ctx);  /* the argument at fault for OG_ERR_INVALID_ARG, else "" */
-const char *og_last_kernel(og_ctx *ctx);          /* name of the last kernel launched on ctx (a product: its class) */
+const char *og_last_kernel(og_ctx *ctx);          /* name of the last kernel launched on ctx (of a product in two launches: the first's) */
 const char *og_version(void);
 
 /* ------------------------------------------------------------------ benchmark and test utilities

@@ -484,17 +484,22 @@ bool tiled_uses_large(int32_t M, int32_t N, int32_t batch)
     return big >= 200;
 }
 
+const char *tiled_kernel_name(const GemmArgs &g)
+{
+    if (!tiled_fast_ok(g)) return "mfma-i8-generic128x128x64";
+    if (direct_ok(g)) return direct_uses_large(g) ? "mfma-i8-direct256x256x64" : "mfma-i8-direct128x128x64";
+    return (g.flags & OG_GEMM_LARGE_TILE) || tiled_uses_large(g.M, g.N, g.batch) ? "mfma-i8-tile256x256x64" : "mfma-i8-tile128x128x128";
+}
+
 hipError_t launch_gemm_tiled(const GemmArgs &g, hipStream_t s, const char **kernel)
 {
     if (!tiled_fast_ok(g)) return launch_gemm_generic(g, s, kernel);
     const bool trans_b = g.flags & OG_GEMM_TRANSPOSE_B;
     const bool large = (g.flags & OG_GEMM_LARGE_TILE) || tiled_uses_large(g.M, g.N, g.batch);
     if (direct_ok(g)) return launch_gemm_direct(g, s, kernel, direct_uses_large(g));
-    if (large) {
-        *kernel = "mfma-i8-tile256x256x64";
+    *kernel = tiled_kernel_name(g);
+    if (large)
         return trans_b ? launch_tiled_cfg<256, 256, 64, 2, 2, true>(g, s) : launch_tiled_cfg<256, 256, 64, 2, 2, false>(g, s);
-    }
-    *kernel = "mfma-i8-tile128x128x128";
     return trans_b ? launch_tiled_cfg<128, 128, 128, 2, 2, true>(g, s) : launch_tiled_cfg<128, 128, 128, 2, 2, false>(g, s);
 }
 

@@ -643,9 +643,21 @@ uint32_t waves_range_groups(const GemmArgs &g, const WavesPlan &p)
     return (uint32_t)std::min<int64_t>(n, int64_t(1) << 30);
 }
 
-hipError_t launch_gemm_waves(const GemmArgs &g, const WavesPlan &p, const Workspace &ws, hipStream_t s,
-                             const ConvView *cv)
+// The tile's rows, columns and waves; "-splitk" where K is cut into slices.
+const char *waves_name(const WavesPlan &p, bool conv)
 {
+#define OG_N(tile) {{"mfma-i8-waves" tile, "mfma-i8-waves" tile "-splitk"}, {"conv-waves" tile, "conv-waves" tile "-splitk"}}
+    static const char *const names[][2][2] = {OG_N("16x16x4"), OG_N("16x32x4"), OG_N("16x64x4"), OG_N("16x64x1"), OG_N("16x128x4"),
+                                              OG_N("32x32x2"), OG_N("32x32x4"), OG_N("32x64x4"), OG_N("32x64x1"),
+                                              OG_N("64x64x4"), OG_N("64x64x2")};
+#undef OG_N
+    return names[p.shape][conv][p.slices > 1];
+}
+
+hipError_t launch_gemm_waves(const GemmArgs &g, const WavesPlan &p, const Workspace &ws, hipStream_t s,
+                             const char **kernel, const ConvView *cv)
+{
+    *kernel = waves_name(p, cv != nullptr);
     GemmArgs a = g;
     if (p.slices > 1) {
         a.C = ws.partials;

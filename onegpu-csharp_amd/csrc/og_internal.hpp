@@ -79,6 +79,7 @@ const char *gemm_kernel_name(GemmKernel k);
 hipError_t launch_gemm_portable(const GemmArgs &g, hipStream_t s, const char **kernel);
 // The MFMA tiled product: the aligned kernel when tiled_fast_ok(g), else the generic one.
 hipError_t launch_gemm_tiled(const GemmArgs &g, hipStream_t s, const char **kernel);
+const char *tiled_kernel_name(const GemmArgs &g);   // as launch_gemm_tiled reports it
 hipError_t launch_gemm_generic(const GemmArgs &g, hipStream_t s, const char **kernel);
 // The kernel fed by LDS DMA (16-byte aligned operands, K a multiple of 64), 256 x 256 tiles for large products, else
 // 128 x 128; launch_gemm_tiled picks it when it applies.
@@ -124,7 +125,8 @@ struct ConvView {
     uint32_t magic_taps, magic_kw;           // floor(2^32 / d) + 1: umulhi(x, magic) = x / d for x d < 2^32, d > 1
 };
 hipError_t launch_gemm_waves(const GemmArgs &g, const WavesPlan &p, const Workspace &ws, hipStream_t s,
-                             const ConvView *cv = nullptr);
+                             const char **kernel, const ConvView *cv = nullptr);
+const char *waves_name(const WavesPlan &p, bool conv);   // as launch_gemm_waves reports it
 bool tiled_uses_large(int32_t M, int32_t N, int32_t batch);
 // Few rows (M <= 16), B stored K x N: split-k partial sums into ws.partials, then a pass that adds them up, corrects for
 // the zero points and applies the epilogue. `slices` is the split chosen by skinny_slices().

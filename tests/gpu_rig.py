@@ -102,13 +102,38 @@ def run_int32(d, gemm, c: cases.Case, seed: int, want: np.ndarray | None = None)
 
 # The options of each configuration: as chosen, portable, and the test hooks that force each kernel.
 CONFIG_OPTIONS = {"default": {}, "portable": {"AllowPackedDot": False}, "tiled only": {"Tile": 64},
-                  "split k": {"Tile": 32}, "large tile": {"Tile": 256}}
+                  "split k": {"Tile": 32}, "large tile": {"Tile": 256}, "two launches": {"FewRowsOneLaunch": False}}
 
 
 def configs(d, all_: bool, **extra):
     """Int8Tests.Configs (Int8Tests.cs:23-34); `extra` adds options (FusedRequantize) to every configuration."""
     names = ["default", "portable"] + (["tiled only", "split k", "large tile"] if all_ else [])
     return [(n, og.Int8Gemm(d, og.Int8GemmOptions(**CONFIG_OPTIONS[n], **extra))) for n in names]
+
+
+def run_noalloc_int32(d, c: cases.Case, seed: int, want: np.ndarray | None = None) -> tuple[int, str]:
+    """run_int32's product through og_int8_gemm_noalloc, whose few-rows products of 16 column slabs and more all take the
+    one-launch kernel; returns (mismatches, kernel run)."""
+    L, p = abi(), c.p
+    data = cases.case_data(c, seed)
+    if want is None:
+        want = cases.reference_sums(c, data)
+    out = np.full(want.size + 2, SENTINEL, np.int32)
+    bc, ba, bb = d.CreateBuffer(out), d.CreateBuffer(as_u8(data["a"])), d.CreateBuffer(as_u8(data["b"]))
+    flags = (0x1 if c.a_signed else 0) | (0x2 if c.b_signed else 0) | (0x4 if p.TransposeB else 0)
+    none, zps = L.Buf(None, 0), []
+    for zp, mode, here, each in ((data["za"], c.za_mode, 0x8, 0x10), (data["zb"], c.zb_mode, 0x20, 0x40)):
+        zps.append(None if zp is None else d.CreateBuffer(as_u8(zp)))
+        flags |= 0 if zp is None else here | (each if mode == 2 else 0)
+    prm = L.GemmParams(M=p.M, N=p.N, K=p.K, Lda=p.Lda, Ldb=p.Ldb, Flags=flags, StrideA=p.StrideA, StrideB=p.StrideB,
+                       StrideC=p.M * p.N)
+    fn = L.og_int8_gemm_noalloc
+    fn.argtypes, fn.restype = L.og_int8_gemm.argtypes, ctypes.c_int
+    check(fn(d.Context, ctypes.byref(prm), p.Batch, binding(ba), binding(bb), binding(bc),
+             *(none if z is None else binding(z) for z in zps), none, none, none), d)
+    kernel = L.og_last_kernel(d.Context).decode()
+    got = bc.Read()
+    return int(np.count_nonzero(got[:want.size] != want)) + int(np.count_nonzero(got[want.size:] != SENTINEL)), kernel
 
 
 _ABI = None

@@ -70,11 +70,13 @@ def _run_case(d, conv, c: dict, seed: int) -> tuple[int, str]:
 
 
 def _configs(d):
-    """ConvIntegerTests.Check's two families (ConvIntegerTests.cs:197-221), plus depthwise through the column matrix."""
+    """ConvIntegerTests.Check's two families (ConvIntegerTests.cs:197-221), plus depthwise through the column matrix, and
+    every convolution through it to the tiled products."""
     out = [("mfma", og.ConvIntegerKernels(d)), ("portable", og.ConvIntegerKernels(d, og.Int8GemmOptions(AllowPackedDot=False)))]
     k = og.ConvIntegerKernels(d)
     k.DirectDepthwise = False
     out.append(("mfma, depthwise as products", k))
+    out.append(("column matrix, tiled", og.ConvIntegerKernels(d, og.Int8GemmOptions(Tile=64))))
     return out
 
 
@@ -118,7 +120,7 @@ def test_model_shapes_are_bit_exact(index):
     # WhisperStemIsBitExact and ResNetShapesAreBitExact (ConvIntegerTests.cs:277-307).
     d = device()
     c = cases.conv_model_cases()[index]
-    for name, conv in _configs(d)[:2]:
+    for name, conv in _configs(d)[:2] + _configs(d)[3:]:
         say(f"conv [{name}] {c['name']}")
         bad, kern = _run_case(d, conv, c, 500 + index)
         say(f"ROW conv integer {c['name']} [{name}, {kern}]: {bad} elements differ")
@@ -131,7 +133,7 @@ def test_padded_depth_with_groups_and_chunks():
     # caller scratch that holds 1 or 2 images (a batch of 3 runs in chunks, the later chunks reusing the weight copy)
     # at an offset that leaves the copy to align its own start, and every zero-point form.
     d = device()
-    conv = og.ConvIntegerKernels(d)
+    conv = og.ConvIntegerKernels(d, og.Int8GemmOptions(Tile=64))   # the column matrix and the tiled kernels
     base = cases.conv_problem(3, 80, 9, 11, 48, 3, 3, stride=1, pad=1, groups=2)   # K = 40 * 9 = 360 -> 384
     seed = 900
     for scratch_images, xs, ws, xzm, wzm in ((1, False, True, 1, 2), (2, True, False, 1, 1), (0, False, False, 0, 2),

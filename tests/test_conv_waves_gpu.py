@@ -45,3 +45,4 @@ def test_convolutions_without_a_column_matrix_are_bit_exact(index):
         say(f"{c['name']} pads {pads} dilation {dil} groups {groups} signed {c['xs']}/{c['ws']} zp {c['xzm']}/{c['wzm']}")
         bad, kern = _run_case(d, conv, c, 7000 + 10 * index + s)
         assert bad == 0, f"{c['name']}: {bad} elements differ ({kern})"
+        assert kern.startswith("conv-waves" if kh * kw > 1 else "mfma-i8-waves"), kern

@@ -541,27 +541,49 @@ def test_kernel_choice_is_reported():
         lib.og_int8_gemm_kernel_name(ctypes.byref(GemmParams(**kw)), 1, out, 64)
         return out.value.decode()
 
+    def tiled(**kw):   # OG_GEMM_NO_SKINNY: the tiled kernels, whatever the size
+        return name(**{**kw, "Flags": kw.get("Flags", 0) | 0x800})
+
     assert name(M=4096, N=4096, K=4096) == "mfma-i8-direct256x256x64"
-    assert name(M=256, N=256, K=64) == "mfma-i8-direct128x128x64"
-    assert name(M=256, N=256, K=96) == "mfma-i8-tile128x128x128"          # K % 64 != 0: register-staged
-    assert name(M=256, N=256, K=64, Ldb=260) == "mfma-i8-tile128x128x128"   # rows of B 4-byte aligned only
-    assert name(M=256, N=256, K=64, Lda=72) == "mfma-i8-generic128x128x64"  # rows of A 8-byte aligned only
+    assert tiled(M=256, N=256, K=64) == "mfma-i8-direct128x128x64"
+    assert tiled(M=256, N=256, K=96) == "mfma-i8-tile128x128x128"          # K % 64 != 0: register-staged
+    assert tiled(M=256, N=256, K=64, Ldb=260) == "mfma-i8-tile128x128x128"   # rows of B 4-byte aligned only
+    assert tiled(M=256, N=256, K=64, Lda=72) == "mfma-i8-generic128x128x64"  # rows of A 8-byte aligned only
     assert name(M=256, N=256, K=64, Flags=0x2000) == "mfma-i8-direct256x256x64"
     assert name(M=1, N=11008, K=4096) == "mfma-i8-rows16-xcd"             # 43 slabs: one launch
     assert name(M=1, N=11008, K=4096, Flags=0x8000) == "mfma-i8-rows16-tiles"   # OG_GEMM_TWO_PASS
-    assert name(M=1, N=1536, K=768) == "mfma-i8-rows16-tiles"             # 12 slabs of 128: under two an XCD
-    assert name(M=16, N=4096, K=4096) == "mfma-i8-rows16-xcd"
-    assert name(M=1, N=11008, K=4100) == "mfma-i8-rows16-splitk"          # K % 16 != 0: not tiled
-    assert name(M=1, N=11008, K=4096, Flags=0x4000) == "mfma-i8-rows16-splitk"
-    assert name(M=1, N=11000, K=4096) == "mfma-i8-rows16-splitk"          # N % 16 != 0: not tiled
-    assert name(M=16, N=11008, K=4096).startswith("mfma-i8-rows16")
+    assert name(M=1, N=1536, K=4096) == "mfma-i8-rows16-tiles"            # 12 slabs of 128: under two an XCD
+    assert name(M=1, N=11008, K=4096, Flags=0x4000) == "mfma-i8-rows16-splitk"   # OG_GEMM_NO_STREAM
+    assert name(M=1, N=64, K=64, Flags=0x4000) == "mfma-i8-rows16-direct"        # one slice
+    assert name(M=1, N=11000, K=4096, Flags=0x5000) == "mfma-i8-rows16-splitk"   # and OG_GEMM_NO_DIRECT
+    assert name(M=1, N=10, K=4096) == "mfma-i8-rows16-splitk"             # under 16 columns: not the waves kernel's
     # Transposed B takes the tiled kernels; 86 tiles of 128 over 64 stages of K split into 3 slices.
-    assert name(M=1, N=11008, K=4096, Flags=0x4) == "mfma-i8-direct128x128x64-splitk"
-    assert name(M=256, N=256, K=2304) == "mfma-i8-direct128x128x64-splitk"   # 4 tiles, 36 stages
+    assert tiled(M=1, N=11008, K=4096, Flags=0x4) == "mfma-i8-direct128x128x64-splitk"
+    assert tiled(M=256, N=256, K=2304) == "mfma-i8-direct128x128x64-splitk"   # 4 tiles, 36 stages
     assert name(M=1024, N=3072, K=768) == "mfma-i8-direct128x128x64"          # 192 tiles: no split
     assert name(M=2048, N=3072, K=768) == "mfma-i8-direct128x128x64"          # 384 tiles: two workgroups a CU
-    assert name(M=256, N=256, K=448) == "mfma-i8-direct128x128x64"            # 7 stages: too short to split
+    assert tiled(M=256, N=256, K=448) == "mfma-i8-direct128x128x64"           # 7 stages: too short to split
     assert name(M=1, N=11008, K=4096, Flags=0x400) == "portable-tile64x64x16"
+    # The waves kernel, named for its tile's rows, columns and waves.
+    assert name(M=256, N=256, K=64) == "mfma-i8-waves32x32x2"
+    assert name(M=256, N=256, K=2304) == "mfma-i8-waves32x32x4"               # a longer walk on few tiles
+    assert name(M=130, N=128, K=4096) == "mfma-i8-waves32x32x4-splitk"        # 20 tiles, 64 steps: slices of K
+    assert name(M=512, N=1024, K=1024) == "mfma-i8-waves32x64x4"              # 512 tiles of 32 x 32, 256 of 32 x 64
+    assert name(M=1024, N=768, K=1536) == "mfma-i8-waves64x64x4"
+    assert name(M=2000, N=2001, K=2003) == "mfma-i8-waves64x64x2"             # unaligned, past one round of the CUs
+    assert name(M=1, N=1536, K=768) == "mfma-i8-waves16x16x4"
+    assert name(M=1, N=51865, K=768) == "mfma-i8-waves16x64x1"
+    assert name(M=16, N=11008, K=4096) == "mfma-i8-waves16x64x4"
+    # A K of 80 steps and more over more tiles than it can be sliced for goes back to the split 128 tile.
+    assert name(M=150, N=1408, K=5120) == "mfma-i8-direct128x128x64-splitk"
+    assert name(M=128, N=1024, K=8192) == "mfma-i8-waves32x64x4-splitk"
+    # Tiles of 256 that are mostly padding, or partial ones with byte sums of A, are left for 128.
+    def wide(m, n, k, batch, flags=0x2):
+        lib.og_int8_gemm_kernel_name(ctypes.byref(GemmParams(M=m, N=n, K=k, Flags=flags, StrideA=m * k, StrideB=k * n)), batch, out, 64)
+        return out.value.decode()
+
+    assert wide(40, 304, 64, 200) == wide(129, 272, 128, 104, 0x2 | 0x60) == "mfma-i8-direct128x128x64"
+    assert wide(256, 256, 64, 200, 0) == wide(250, 512, 64, 101) == "mfma-i8-direct256x256x64"
 
 
 class DqParams(ctypes.Structure):

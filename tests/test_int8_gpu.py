@@ -8,7 +8,7 @@ import pytest
 import cases
 import oracle
 import onegpu_hip as og
-from gpu_rig import CONFIG_OPTIONS, as_i8, as_u8, configs, device, run, run_int32, say, to_problem, binding, abi, check
+from gpu_rig import CONFIG_OPTIONS, as_i8, as_u8, configs, device, run, run_int32, run_noalloc_int32, say, to_problem, binding, abi, check
 
 pytestmark = pytest.mark.gpu
 
@@ -140,14 +140,22 @@ def test_float_and_requantized_forms_are_bit_exact(config):
     assert bad_f + bad_q == 0
 
 
-# Shapes that reach every kernel: few rows on the tiled few-rows kernel (or split k), the 128 and 256 direct kernels
-# (ragged M included), the register-staged 128 tile (K = 96), the generic kernel (unaligned rows), tiny products.
-# The last three reach the one-launch few-rows kernel with its k-slices handed to the finishing tile (16 to 36 column
-# slabs of 2 to 8 row bands), so its epilogues are checked after a real hand-off.
+# Shapes that reach every kernel, each in some configuration (EVERY_KERNEL): few rows on the tiled few-rows kernels (or
+# split k), the waves kernel, the 128 and 256 direct kernels (ragged M included), the register-staged 128 tile (K = 96),
+# the generic kernel (unaligned rows), tiny products. The last three reach the one-launch few-rows kernel with its
+# k-slices handed to the finishing tile (16 to 36 column slabs of 8 to 9 row bands), so its epilogues are checked after
+# a real hand-off.
 REQUANT_KERNEL_SHAPES = [(1, 1, 1), (5, 7, 9), (4, 272, 512), (16, 256, 1024), (64, 64, 96), (33, 257, 77),
                          (128, 384, 384), (130, 256, 512), (2, 8192, 128), (96, 208, 320), (3, 4608, 272),
-                         (3, 4608, 1024), (4, 2048, 4096), (16, 2048, 2048)]
+                         (3, 4608, 1024), (16, 2048, 2048), (3, 4608, 4096), (4, 2048, 4096), (1, 2176, 4112)]
 HANDOFF_SHAPES = REQUANT_KERNEL_SHAPES[-3:]
+EVERY_KERNEL = {
+    "default": {"mfma-i8-rows16-xcd", "mfma-i8-rows16-direct", "mfma-i8-waves16x16x4", "mfma-i8-waves32x32x2"},
+    "portable": {"portable-tile64x64x16"},
+    "tiled only": {"mfma-i8-direct128x128x64", "mfma-i8-tile128x128x128", "mfma-i8-generic128x128x64"},
+    "split k": {"mfma-i8-rows16-splitk"},
+    "large tile": {"mfma-i8-direct256x256x64", "mfma-i8-tile256x256x64"},
+    "two launches": {"mfma-i8-rows16-tiles"}}
 
 
 @pytest.mark.parametrize("fused", [True, False], ids=["one launch", "two passes"])
@@ -172,12 +180,9 @@ def test_requantized_product_on_every_kernel(config, fused):
     say(f"ROW requantized [{config}, {'one launch' if fused else 'two passes'}] wrong bytes {bad}; kernels "
         f"{sorted(kernels)}")
     assert bad == 0
-    if fused and config == "default":
-        assert {"mfma-i8-rows16-tiles", "mfma-i8-rows16-xcd", "mfma-i8-direct128x128x64",
-                "mfma-i8-tile128x128x128", "mfma-i8-generic128x128x64"} <= kernels, kernels
-    if fused and config == "large tile":
-        assert "mfma-i8-direct256x256x64" in kernels, kernels
-    if not fused:
+    if fused:
+        assert EVERY_KERNEL[config] <= kernels, kernels
+    else:
         assert kernels == {"int8-epilogue"}, kernels
 
 
@@ -224,6 +229,7 @@ def test_scaled_float_product_on_every_kernel(config):
             seed += 1
     say(f"ROW scaled float [{config}] wrong values {bad}; kernels {sorted(kernels)}")
     assert bad == 0
+    assert EVERY_KERNEL[config] <= kernels, kernels
 
 
 @pytest.mark.parametrize("fused", [True, False], ids=["one launch", "two passes"])
@@ -401,8 +407,9 @@ def test_products_wider_than_one_grid_axis_are_bit_exact():
 
 
 @pytest.mark.parametrize("config, k, want_kernel", [
-    ("default", 128, "mfma-i8-direct128x128x64"), ("large tile", 128, "mfma-i8-direct256x256x64"),
-    ("default", 96, "mfma-i8-tile128x128x128"), ("large tile", 96, "mfma-i8-tile256x256x64")])
+    ("tiled only", 128, "mfma-i8-direct128x128x64"), ("large tile", 128, "mfma-i8-direct256x256x64"),
+    ("tiled only", 96, "mfma-i8-tile128x128x128"), ("large tile", 96, "mfma-i8-tile256x256x64"),
+    ("default", 128, "mfma-i8-waves32x32x2"), ("default", 96, "mfma-i8-waves32x32x2")])
 def test_padded_rows_of_b_with_a_ragged_width(config, k, want_kernel):
     # B stored K x N in rows of Ldb > N bytes with N not a multiple of 4 (ConvInteger's column matrices have this
     # shape): the final dword of B's last row holds valid columns and padding, and every column must come through.
@@ -429,7 +436,8 @@ def test_padded_rows_of_b_with_a_ragged_width(config, k, want_kernel):
 
 def test_b_ending_at_its_last_valid_byte_takes_another_kernel():
     # The same product through the C ABI with B's buffer declared to end at its last valid byte: the dword-wide reads
-    # of the aligned kernels would leave it, so a kernel with byte-exact reads runs instead, with the same sums.
+    # of the aligned kernels would leave it, so among the tiled kernels (OG_GEMM_NO_SKINNY) the one with byte-exact reads
+    # runs instead, with the same sums; the waves kernel's reads end there by themselves.
     d = device()
     m, n, k, ldb = 200, 750, 128, 752
     rng = np.random.default_rng(5)
@@ -439,35 +447,36 @@ def test_b_ending_at_its_last_valid_byte_takes_another_kernel():
     ba, bb = d.CreateBuffer(a), d.CreateBuffer(b.view(np.int8))
     bc = d.CreateBufferOf(og.ElementType.Int32, m * n)
     L = abi()
-    prm = L.GemmParams(M=m, N=n, K=k, Lda=k, Ldb=ldb, Flags=0x002, StrideC=m * n)
     none = L.Buf(None, 0)
     exact = L.Buf(bb.DevicePointer, (k - 1) * ldb + n)
-    check(L.og_int8_gemm(d.Context, ctypes.byref(prm), 1, binding(ba), exact, binding(bc), none, none, none, none,
-                         none), d)
-    d.WaitIdle()
-    kernel = L.og_last_kernel(d.Context).decode()
-    assert "direct" not in kernel and "tile" not in kernel, kernel
-    assert np.array_equal(bc.Read(), want)
-    check(L.og_int8_gemm(d.Context, ctypes.byref(prm), 1, binding(ba), binding(bb), binding(bc), none, none, none,
-                         none, none), d)
-    d.WaitIdle()
-    assert L.og_last_kernel(d.Context).decode() == "mfma-i8-direct128x128x64"
-    assert np.array_equal(bc.Read(), want)
+    for flags, b_buf, want_kernel in ((0x802, exact, "mfma-i8-generic128x128x64"),
+                                      (0x802, binding(bb), "mfma-i8-direct128x128x64"),
+                                      (0x002, exact, "mfma-i8-waves32x32x2")):
+        say(f"B to its last byte, flags {flags:#x}: {want_kernel}")
+        prm = L.GemmParams(M=m, N=n, K=k, Lda=k, Ldb=ldb, Flags=flags, StrideC=m * n)
+        check(L.og_int8_gemm(d.Context, ctypes.byref(prm), 1, binding(ba), b_buf, binding(bc), none, none, none, none,
+                             none), d)
+        d.WaitIdle()
+        assert L.og_last_kernel(d.Context).decode() == want_kernel
+        assert np.array_equal(bc.Read(), want)
 
 
-# Products whose 128 x 128 grid fills under half the chip and whose K has at least 8 stages: split along K.
-SPLIT_SHAPES = [  # m, n, k, batch, transposed B
-    (256, 256, 2304, 1, False), (200, 384, 1536, 1, False), (128, 256, 2048, 2, False), (1, 11008, 4096, 1, True),
-    (130, 128, 4096, 1, True)]
+# Products split along K on the 128 x 128 direct kernel: its grid fills under half the chip, and K has at least 8 stages.
+# The first five ask for the tiled kernels; the others come there by themselves: a deep K over more tiles than the waves
+# kernel cuts into slices.
+SPLIT_SHAPES = [  # m, n, k, batch, transposed B, options
+    (256, 256, 2304, 1, False, {"Tile": 64}), (200, 384, 1536, 1, False, {"Tile": 64}), (128, 256, 2048, 2, False, {"Tile": 64}),
+    (1, 11008, 4096, 1, True, {"Tile": 64}), (130, 128, 4096, 1, True, {"Tile": 64}),
+    (150, 1408, 5120, 1, False, {}), (100, 1411, 3840, 1, True, {}), (32, 4160, 5120, 1, False, {})]
 
 
-@pytest.mark.parametrize("m, n, k, batch, trans", SPLIT_SHAPES)
-def test_split_k_products_are_bit_exact(m, n, k, batch, trans):
+@pytest.mark.parametrize("m, n, k, batch, trans, opts", SPLIT_SHAPES)
+def test_split_k_products_are_bit_exact(m, n, k, batch, trans, opts):
     # The k slices each apply the zero points to their own range (every correction term is linear in the range);
     # the summing pass adds them and applies the bias and the epilogue: int32, float (scale, float bias), scaled
     # float and requantized outputs, both operand signednesses, zero points per row and column.
     d = device()
-    gemm = og.Int8Gemm(d)
+    gemm = og.Int8Gemm(d, og.Int8GemmOptions(**opts))
     rng = np.random.default_rng(m + n + k)
     a = rng.integers(0, 256, batch * m * k, dtype=np.uint8)
     b = rng.integers(0, 256, batch * n * k, dtype=np.uint8)
@@ -560,7 +569,8 @@ def test_few_rows_kernels_are_bit_exact(config):
     # (partial sums per k-slice, then their sum): one slab or many, one tile per slab or several, K past the last full
     # tile or 64 rows, N past the last full slab, M = 16 (no spare MFMA row), batches, every signedness and zero-point
     # form, configuration 3's shape at M = 1, 4 and 16; one case three times in a row and a smaller M after a larger
-    # one. Aligned operands; the tiled kernel takes K and N multiples of 16, the split-k one the rest.
+    # one. Aligned operands; the tiled kernel takes K and N multiples of 16, the split-k one the rest. "tiles" goes
+    # through og_int8_gemm_noalloc, whose one-launch products stay on that kernel at every size.
     d = device()
     opts = {"tiles": og.Int8GemmOptions(), "tiles two launches": og.Int8GemmOptions(FewRowsOneLaunch=False),
             "split k": og.Int8GemmOptions(Tile=32)}[config]
@@ -579,22 +589,24 @@ def test_few_rows_kernels_are_bit_exact(config):
         one_launch = config == "tiles" and batch * ((n + 127) // 128) >= 16
         for rep in range(3 if i == 2 or i == 8 else 1):
             say(f"{config} case {c.name} signed {a_s}/{b_s} zp {za_mode}/{zb_mode} rep {rep}")
-            bad, kernel = run_int32(d, gemm, c, 100 + i)
+            bad, kernel = run_noalloc_int32(d, c, 100 + i) if config == "tiles" else run_int32(d, gemm, c, 100 + i)
             d.WaitIdle()   # reports a one-launch product whose parts never arrived
             if bad:
                 say(f"  {kernel}: {bad} wrong")
             kernels.add(kernel)
-            if tiled:
-                assert kernel == ("mfma-i8-rows16-xcd" if one_launch else "mfma-i8-rows16-tiles"), kernel
-            else:
+            if config == "split k":
                 assert kernel in ("mfma-i8-rows16-splitk", "mfma-i8-rows16-direct"), kernel
+            elif tiled and (one_launch or config == "tiles two launches"):
+                assert kernel == ("mfma-i8-rows16-xcd" if one_launch else "mfma-i8-rows16-tiles"), kernel
+            else:   # too few slabs to hand over, or rows off 16 bytes
+                assert kernel.startswith(("mfma-i8-waves", "mfma-i8-rows16-direct")), kernel
             bad_total += bad
     for vec in (False, True):
         say(f"{config} float vec {vec}")
         bad_total += _float_case(d, gemm, 4, 256, 128, vec, True, True, 77 + vec)
         bad_total += _float_case(d, gemm, 16, 1024, 512, vec, False, True, 79 + vec)
         bad_total += _float_case(d, gemm, 3, 8192, 192, vec, True, True, 81 + vec)
-        # Column slabs of 8, 2 and 4 row bands: the finishing tile's float store after a real hand-off.
+        # Column slabs of 8 and 9 row bands: the finishing tile's float store after a real hand-off.
         for j, (m, n, k) in enumerate(HANDOFF_SHAPES):
             bad_total += _float_case(d, gemm, m, n, k, vec, j != 1, j != 0, 83 + 2 * j + vec)
             if config == "tiles":
@@ -608,8 +620,8 @@ def test_c3_matmul_integer_to_float_few_rows(m):
     # Configuration 3 as the decode layer runs it: DynamicQuantizeLinear of N(0, 1) activations [m x 4096], then
     # MatMulIntegerToFloat with int8 weights [4096 x 11008] quantized symmetric per column from N(0, 0.02), the column
     # scale fl(actScale * wScale[n]) made in the product's epilogue (EncodeFloatScaled) and, as the reference chains
-    # it, the scale vector made first (EncodeFloat). The one-launch few-rows kernel hands 8 k-slices of each of 86
-    # column slabs to the slab's finishing tile. Against the oracle: DQ's bytes, scale and zero point, then every
+    # it, the scale vector made first (EncodeFloat). At m = 1 and 4 the one-launch few-rows kernel hands 8 k-slices of each
+    # of 86 column slabs to the slab's finishing tile. Against the oracle: DQ's bytes, scale and zero point, then every
     # output bit.
     K, N = 4096, 11008
     d = device()
@@ -642,7 +654,7 @@ def test_c3_matmul_integer_to_float_few_rows(m):
             run(d, lambda e: (e.RecordScaleProduct(bs, bws, N, bsc),
                               gemm.EncodeFloat(e, p, by, bq, bc, og.Int8Operand(bsc, 0, True), og.Int8Operand(bz, 0))))
         d.WaitIdle()
-        assert d.LastKernel == "mfma-i8-rows16-xcd", d.LastKernel
+        assert d.LastKernel == ("mfma-i8-rows16-xcd" if m <= 4 else "mfma-i8-waves16x64x4"), d.LastKernel
         got = bc.Read()
         bad = int(np.count_nonzero(got.view(np.uint32) != want.view(np.uint32)))
         say(f"ROW c3 MatMulIntegerToFloat m {m} ({form}): {bad} wrong values")
@@ -798,12 +810,14 @@ LARGE_K_CASES = [
      "mfma-i8-direct256x256x64"),
     ("256 tile ping-pong, A's zero point per row", 256, 256, 40960, False, True, 2, 0, "large tile",
      "mfma-i8-direct256x256x64"),
-    ("128 tile split along K", 128, 128, 40960, False, False, 1, 2, "default", "mfma-i8-direct128x128x64"),
+    ("128 tile split along K", 128, 128, 40960, False, False, 1, 2, "tiled only", "mfma-i8-direct128x128x64-splitk"),
     ("128 tile whole, C misaligned for the staged store", 1152, 1920, 40960, False, False, 2, 2, "default",
      "mfma-i8-direct128x128x64"),
     ("register-staged tile, K not a multiple of 64", 64, 64, 40976, False, False, 2, 1, "tiled only",
      "mfma-i8-tile128x128x128"),
     ("generic kernel, unaligned rows", 64, 64, 40961, False, False, 1, 2, "tiled only", "mfma-i8-generic128x128x64"),
+    ("waves in slices of K, both zero points", 64, 64, 40961, False, False, 1, 2, "default", "mfma-i8-waves32x32x4-splitk"),
+    ("waves, one column tile of K x N", 1, 16, 40961, False, False, 2, 2, "default", "mfma-i8-waves16x16x4"),
     ("few rows, one launch", 4, 2048, 40960, False, False, 1, 2, "default", "mfma-i8-rows16-xcd"),
     # 127 k-slices a column slab, the most its 7-bit count fields take; 128 go to the two-launch kernel.
     ("few rows, one launch, 127 k-slices", 3, 2048, 127 * 512, False, True, 2, 0, "default", "mfma-i8-rows16-xcd"),

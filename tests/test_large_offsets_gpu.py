@@ -19,24 +19,27 @@ STRIDE = 3 << 29   # 1.5 GiB between batch entries: entry 2 starts 3 GiB in, ent
 BATCH = 4
 REGION = 4 << 20   # room for the largest entry below
 A_INT8, B_INT8, TRANS_B, ZA, ZA_ROW, ZB, ZB_COL = 0x1, 0x2, 0x4, 0x8, 0x10, 0x20, 0x40
-PORTABLE, NO_SKINNY, LARGE_TILE, TWO_PASS = 0x400, 0x800, 0x2000, 0x8000
+PORTABLE, NO_SKINNY, NO_DIRECT, LARGE_TILE, NO_STREAM, TWO_PASS = 0x400, 0x800, 0x1000, 0x2000, 0x4000, 0x8000
 
-# (label, m, n, k, flags, the kernel the product takes)
+# (label, m, n, k, flags, the kernel the product takes); the flags keep the product on it where the waves kernel would run.
 CASES = [
-    ("direct 128", 128, 256, 256, B_INT8 | ZA | ZA_ROW, "mfma-i8-direct128x128x64"),
-    ("direct 128 split along K", 128, 128, 2048, B_INT8 | ZA, "mfma-i8-direct128x128x64-splitk"),
+    ("direct 128", 128, 256, 256, B_INT8 | ZA | ZA_ROW | NO_SKINNY, "mfma-i8-direct128x128x64"),
+    ("direct 128 split along K", 128, 128, 2048, B_INT8 | ZA | NO_SKINNY, "mfma-i8-direct128x128x64-splitk"),
     ("direct 256, both zero points", 256, 256, 256, ZA | ZB | ZB_COL | NO_SKINNY | LARGE_TILE,
      "mfma-i8-direct256x256x64"),
     ("direct 256 ping-pong", 256, 256, 256, B_INT8 | ZA | ZA_ROW | NO_SKINNY | LARGE_TILE, "mfma-i8-direct256x256x64"),
     ("direct 256, B stored N x K", 256, 256, 256, B_INT8 | TRANS_B | ZA | NO_SKINNY | LARGE_TILE,
      "mfma-i8-direct256x256x64"),
-    ("register-staged tile", 64, 64, 208, A_INT8 | ZA | ZB, "mfma-i8-tile128x128x128"),
-    ("generic, unaligned rows", 64, 64, 200, ZA | ZB | ZB_COL, "mfma-i8-generic128x128x64"),
-    ("few rows, one launch", 2, 2048, 1024, B_INT8 | ZA, "mfma-i8-rows16-xcd"),
+    ("register-staged tile", 64, 64, 208, A_INT8 | ZA | ZB | NO_SKINNY, "mfma-i8-tile128x128x128"),
+    ("generic, unaligned rows", 64, 64, 200, ZA | ZB | ZB_COL | NO_SKINNY, "mfma-i8-generic128x128x64"),
+    ("few rows, one launch", 2, 512, 4096, B_INT8 | ZA, "mfma-i8-rows16-xcd"),
     ("few rows, two launches", 2, 2048, 1024, B_INT8 | ZA | TWO_PASS, "mfma-i8-rows16-tiles"),
-    ("few rows split k", 3, 1000, 2000, B_INT8 | ZA | ZB, "mfma-i8-rows16-splitk"),
-    ("few rows, one k slice", 2, 1000, 64, B_INT8 | ZA | ZB, "mfma-i8-rows16-direct"),
+    ("few rows split k", 3, 1000, 2000, B_INT8 | ZA | ZB | NO_STREAM | NO_DIRECT, "mfma-i8-rows16-splitk"),
+    ("few rows, one k slice", 2, 1000, 64, B_INT8 | ZA | ZB | NO_STREAM, "mfma-i8-rows16-direct"),
     ("portable", 64, 64, 256, A_INT8 | ZA | ZB | ZB_COL | PORTABLE, "portable-tile64x64x16"),
+    ("waves", 64, 64, 200, ZA | ZB | ZB_COL, "mfma-i8-waves32x32x2"),
+    ("waves, B stored N x K off a dword", 63, 65, 201, B_INT8 | TRANS_B | ZA | ZB, "mfma-i8-waves32x32x2"),
+    ("waves in slices of K", 40, 72, 4097, B_INT8 | ZA, "mfma-i8-waves32x32x4-splitk"),
 ]
 
 

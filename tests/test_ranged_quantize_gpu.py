@@ -22,16 +22,20 @@ pytestmark = pytest.mark.gpu
 
 # (label, m, n, k, batch, options, the kernel the product takes, whether that kernel writes the ranges itself)
 CASES = [
-    ("direct 128", 256, 384, 512, 1, {}, "mfma-i8-direct128x128x64", True),
-    ("direct 128, batch 3", 128, 256, 320, 3, {}, "mfma-i8-direct128x128x64", True),
+    ("direct 128", 256, 384, 512, 1, {"Tile": 64}, "mfma-i8-direct128x128x64", True),
+    ("direct 128, batch 3", 128, 256, 320, 3, {"Tile": 64}, "mfma-i8-direct128x128x64", True),
     ("configuration 2, layer 1", 1024, 3072, 768, 1, {}, "mfma-i8-direct128x128x64", True),
-    ("direct 128, ragged", 200, 144, 192, 1, {}, "mfma-i8-direct128x128x64", True),
-    ("split k", 256, 256, 2304, 1, {}, "mfma-i8-direct128x128x64-splitk", True),
-    ("split k, ragged", 200, 144, 1536, 1, {}, "mfma-i8-direct128x128x64-splitk", True),
+    ("direct 128, ragged", 200, 144, 192, 1, {"Tile": 64}, "mfma-i8-direct128x128x64", True),
+    ("split k", 256, 256, 2304, 1, {"Tile": 64}, "mfma-i8-direct128x128x64-splitk", True),
+    ("split k, ragged", 200, 144, 1536, 1, {"Tile": 64}, "mfma-i8-direct128x128x64-splitk", True),
+    ("split k, as chosen", 150, 1408, 5120, 1, {}, "mfma-i8-direct128x128x64-splitk", True),
     ("few rows, one launch", 4, 2048, 4096, 1, {}, "mfma-i8-rows16-xcd", True),
-    ("few rows, one launch, 16 rows", 16, 4608, 1024, 1, {}, "mfma-i8-rows16-xcd", True),
+    ("waves, 16 rows", 16, 4608, 1024, 1, {}, "mfma-i8-waves16x32x4", True),
+    ("waves, batch 3", 128, 256, 320, 3, {}, "mfma-i8-waves32x32x2", True),
+    ("waves, ragged", 200, 144, 192, 1, {}, "mfma-i8-waves32x32x2", True),
+    ("waves in slices of K", 40, 72, 4096, 1, {}, "mfma-i8-waves32x32x4-splitk", True),
     ("256 tile (range pass)", 512, 512, 256, 1, {"Tile": 256}, "mfma-i8-direct256x256x64", False),
-    ("register-staged tile (range pass)", 64, 64, 96, 1, {}, "mfma-i8-tile128x128x128", False),
+    ("register-staged tile (range pass)", 64, 64, 96, 1, {"Tile": 64}, "mfma-i8-tile128x128x128", False),
     ("few rows, two launches (range pass)", 3, 2048, 512, 1, {"FewRowsOneLaunch": False}, "mfma-i8-rows16-tiles", False),
     ("portable (range pass)", 70, 90, 100, 1, {"AllowPackedDot": False}, "portable-tile64x64x16", False),
 ]

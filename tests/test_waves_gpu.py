@@ -21,16 +21,21 @@ SHAPES = [(1, 16, 16, 1), (16, 17, 63, 1), (3, 385, 65, 1), (15, 250, 129, 3),  
           (1, 20001, 96, 1), (4, 2051, 47, 17),                                       # 16 x 128, or one wave
           (2, 200, 8200, 1), (16, 321, 6500, 1), (1, 1537, 4100, 1),                  # slices of a deep K
           (17, 33, 16, 1), (31, 95, 383, 2), (65, 47, 1601, 1), (40, 40, 3600, 1),    # 32 x 32, two and four waves, slices
-          (129, 1100, 321, 1), (33, 2049, 257, 1),                                    # 32 x 64
-          (33, 6001, 100, 1), (300, 700, 97, 3),                                      # 64 x 64
+          (60, 1057, 5121, 1), (70, 500, 5150, 2), (90, 1999, 5153, 1), (100, 1000, 5184, 2),   # 32 x 64, 64 x 64 in slices
+          (129, 1100, 321, 1), (33, 2049, 257, 1), (33, 6001, 100, 1),                # 32 x 32 on all CUs, 32 x 64
+          (300, 700, 97, 3),                                                          # 64 x 64
           (333, 65, 95, 60), (257, 500, 33, 40), (500, 1025, 650, 2), (30, 2100, 130, 20)]   # more than one round
+
+# The instances that these shapes run off a dword: tile and waves, "-splitk" in slices of K (of a deep K x N alone at 16 rows).
+INSTANCES = {"16x16x4", "16x32x4", "16x64x4", "16x64x1", "32x32x2", "32x32x4", "32x32x4-splitk", "32x64x4", "32x64x4-splitk",
+             "32x64x1", "64x64x4", "64x64x4-splitk", "64x64x2"}
 
 
 @pytest.mark.parametrize("trans", [False, True], ids=["K x N", "N x K"])
 def test_sums_are_bit_exact(trans):
     d = device()
     gemm = og.Int8Gemm(d)
-    bad_total = 0
+    bad_total, kernels = 0, set()
     for i, (m, n, k, batch) in enumerate(SHAPES):
         for v in range(2):
             off, extra = (0, 0) if v == 0 else (1 + i % 3, 1 + (i + 1) % 5)   # rows on, and off, a dword
@@ -41,11 +46,15 @@ def test_sums_are_bit_exact(trans):
             bad, kernel = run_int32(d, gemm, c, 500 + i)
             if bad:
                 say(f"  {kernel}: {bad} wrong")
+            if v == 1:
+                kernels.add(kernel)
             bad_total += bad
     assert bad_total == 0
+    assert kernels == {"mfma-i8-waves" + i for i in INSTANCES | (set() if trans else {"16x128x4", "16x64x4-splitk"})}
 
 
-@pytest.mark.parametrize("m, n, k", [(7, 385, 129), (40, 70, 333), (200, 300, 97), (33, 40, 3600)])
+@pytest.mark.parametrize("m, n, k", [(7, 385, 129), (40, 70, 333), (200, 300, 97), (33, 40, 3600), (60, 1057, 5121),
+                                     (90, 1999, 5153), (100, 2000, 5184)])
 def test_float_ranged_and_requantized_stores(m, n, k):
     # Whole 16-byte pieces of C's rows (n % 4 == 0) and single values, with and without slices.
     d = device()
@@ -73,6 +82,7 @@ def test_float_ranged_and_requantized_stores(m, n, k):
     assert r[:, 0].min() == want.min() and r[:, 1].max() == want.max()
     say(f"waves stores {m}x{n}x{k}: requantized")
     run(d, lambda e: gemm.EncodeRequantized(e, p, ba, bb, y, og.Int8Operand(bm, 0, True), 131, zpa, None, vec(bi)))
+    assert d.LastKernel.startswith("mfma-i8-waves"), d.LastKernel
     assert np.array_equal(y.Read()[:m * n], oracle.requant_array(sums, n, mult, True, 131, True, ib))
 
 
@@ -84,7 +94,7 @@ def test_a_grid_of_tiles_for_the_xcds(m, n, k):
     c = cases.Case(f"waves grid {m}x{n}x{k}", cases.problem(m, n, k), False, True, 2, 1)
     say(c.name)
     bad, kernel = run_int32(d, og.Int8Gemm(d), c, m + n)
-    assert bad == 0, kernel
+    assert bad == 0 and kernel == "mfma-i8-waves64x64x4", (bad, kernel)
 
 
 def test_a_grid_of_tiles_records_every_range():
