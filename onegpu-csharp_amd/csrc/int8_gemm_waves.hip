@@ -19,6 +19,7 @@
 //  - ksplit > 1: blockIdx also picks a slice of K; each slice's sums (its zero points applied) go to a dense int32
 //    buffer of [batch * ksplit + slice][M][N] which the summing pass of the split 128 tile adds up.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "og_internal.hpp"
@@ -628,6 +629,35 @@ WavesPlan waves_plan(const GemmArgs &g)
     p.slice_steps = (int32_t)((steps + slices - 1) / slices);
     p.slices = (int32_t)((steps + p.slice_steps - 1) / p.slice_steps);
     return p;
+}
+
+// Past one round of the CUs, an aligned product whose K is no multiple of 64 (or whose rows of B are whole dwords only) has
+// the register-staged tiles (k_gemm_tiled) as the other choice: they start late, read far less a 64-deep step and win where K
+// is deep. Both as fitted to what they measured (us; k in 1024s, kn and nk the two layouts of B):
+//  - waves: 4 and, a round of 1024 tiles of 64 x 64, 13.5 k (14.4 k nk); a partly filled second round costs 26 k; tall results
+//    15% more, for each XCD reads all of A; and B itself at 2 to 3.4 TB/s, by how many rows of tiles read it.
+//  - 256 tiles: 56 + 23 k a round of 256. 128 tiles: 21.5 + 12.5 k (11.9 k nk) a full round of 512, 18.5 + 9.6 k (7.3 k nk) where the
+//    last round gives a CU at most one.
+// 4096 x 4096 x 4080 kn 149 (256 tiles) against 234 us, x 400 66 against 36; 2048 x 4096 x 3088 56 (128) against 80, x 1040 33 against 30;
+// 2000 x 1504 x 4112 56 against 42; 128 x 50304 x 4112 nk 91 against 133.
+bool staged_tile_faster(const GemmArgs &g)
+{
+    const bool nk = g.flags & OG_GEMM_TRANSPOSE_B;
+    const double k = g.K / 1024.0;
+    auto tiles = [&](int64_t t) { return (double)(((g.M + t - 1) / t) * ((g.N + t - 1) / t) * g.batch); };
+    const double n64 = tiles(64), n128 = tiles(128);
+    double slope = n64 <= 1024 ? 13.5 * std::max(0.65, n64 / 1024) : std::max(26.0, 0.0142 * n64);
+    slope *= (nk ? 1.07 : 1.0) * (g.M >= 4 * (int64_t)g.N ? 1.15 : 1.0);
+    const double waves = 4 + k * std::max(slope, (double)g.N * g.batch / (g.M <= 16 ? 3300 : g.M <= 32 ? 2800 : g.M <= 64 ? 2440 : 2000));
+    double staged = 0;
+    if (tiled_uses_large(g.M, g.N, g.batch)) {
+        staged = std::ceil(tiles(256) / 256) * (56 + 23 * k);
+    } else {
+        const double full = std::floor(n128 / 512), rest = n128 - 512 * full;
+        const double two = 21.5 + (nk ? 11.9 : 12.5) * k, one = (18.5 + (nk ? 7.3 : 9.6) * k) * (full > 0 ? 0.85 : 1.0);
+        staged = full * two + (rest > 256 ? two : rest > 0 ? one : 0);
+    }
+    return staged < waves;
 }
 
 int64_t waves_count(const GemmArgs &g, const WavesPlan &p)

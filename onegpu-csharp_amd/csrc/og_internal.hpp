@@ -113,6 +113,7 @@ struct WavesPlan {
 constexpr int64_t kWavesMaxPartials = int64_t(12) << 20;
 bool waves_ok(const GemmArgs &g);
 WavesPlan waves_plan(const GemmArgs &g);
+bool staged_tile_faster(const GemmArgs &g);   // than its tiles past one round, of a product that tiled_fast_ok takes
 uint32_t waves_range_groups(const GemmArgs &g, const WavesPlan &p);   // its workgroups before slicing: one pair each
 int64_t waves_count(const GemmArgs &g, const WavesPlan &p);             // their waves
 // A convolution's column matrix as that kernel reads it straight from the images (g.B the first image's channels of

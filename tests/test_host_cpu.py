@@ -577,6 +577,15 @@ def test_kernel_choice_is_reported():
     # A K of 80 steps and more over more tiles than it can be sliced for goes back to the split 128 tile.
     assert name(M=150, N=1408, K=5120) == "mfma-i8-direct128x128x64-splitk"
     assert name(M=128, N=1024, K=8192) == "mfma-i8-waves32x64x4-splitk"
+    # Aligned, K no multiple of 64, past one round: the register-staged tiles where K is deep, both layouts of B, a B whose
+    # rows are whole dwords only, a tall result, and one round of them alone.
+    for k, want in ((400, "mfma-i8-waves64x64x2"), (4080, "mfma-i8-tile256x256x64")):
+        assert name(M=4096, N=4096, K=k) == name(M=4096, N=4096, K=k, Flags=0x4) == name(M=4096, N=4004, K=k) == want
+    assert name(M=4096, N=2048, K=784) == "mfma-i8-waves64x64x2"
+    assert name(M=4096, N=2048, K=2064) == name(M=8192, N=1024, K=1040) == "mfma-i8-tile128x128x128"
+    assert name(M=2000, N=1504, K=3088) == name(M=300, N=4096, K=2000, Flags=0x4) == "mfma-i8-waves64x64x2"
+    assert name(M=300, N=4096, K=2000) != name(M=128, N=50304, K=4112, Flags=0x4) == "mfma-i8-tile128x128x128"
+    assert name(M=4096, N=4097, K=4099) == "mfma-i8-waves64x64x2"             # unaligned: only the generic kernel is left
     # Tiles of 256 that are mostly padding, or partial ones with byte sums of A, are left for 128.
     def wide(m, n, k, batch, flags=0x2):
         lib.og_int8_gemm_kernel_name(ctypes.byref(GemmParams(M=m, N=n, K=k, Flags=flags, StrideA=m * k, StrideB=k * n)), batch, out, 64)
