@@ -631,6 +631,27 @@ WavesPlan waves_plan(const GemmArgs &g)
     return p;
 }
 
+// Few rows, B stored K x N. The few-rows kernels request all of B at once, which is what HBM answers fastest, and then hand
+// their parts over, which costs more the more rows there are; here a wave walks its steps one memory latency after the
+// other, with a few in flight. So the line is a depth that grows with the rows and with the columns (more waves to hide
+// a latency, up to one round of the CUs), and rows of B that are multiples of 1 KiB, which keep to few of the memory
+// channels, draw it in. It lies where the two are equal in the mean of B from HBM and B from the Infinity Cache (us, few-rows
+// kernel against this one):
+//   1 x 4096 x 1280     from HBM 7.2, 6.7    from the cache 6.9, 6.4      16 x 4096 x 4096    11.5, 13.8    10.9, 10.4
+//   1 x 4096 x 3584              8.8, 12.1             7.9, 9.2           16 x 11008 x 4096   16.7, 15.0    16.1, 11.0
+//   5 x 8192 x 4096              13, 16                 12, 11.5          16 x 3072 x 5120    12, 16        -
+// Past one round the walk is one wave's alone: 40960 columns of 3072, one row, 27 against 39 us; of 768, 13 against 13. A
+// depth of at most 512 is one part, with nothing to hand over: 1 x 28672 x 512 8.0 against 8.5.
+bool waves_few_rows(const GemmArgs &g)
+{
+    const int64_t cols = (int64_t)g.N * g.batch, slabs = (int64_t)((g.N + 127) / 128) * g.batch;
+    if (slabs < 16) return g.K <= 2560;   // the two-launch form: 1 x 1024 x 1024 7.7 against 5.3 us, 8 x 1024 x 4096 8.1 against 11.6 from HBM
+    if (g.M <= 4 && g.K >= 4096) return false;
+    if (g.M <= 8 && g.K > 256 && g.K <= 512 && cols > 16384) return false;
+    if (!waves_plan(g).one_round) return g.M > 8 ? g.K <= 1024 : g.K <= (cols <= 65536 ? 768 : 256);
+    return g.K <= 5120 && g.K <= 1536 + 128 * g.M + std::min<int64_t>(cols, 32768) / 32 + (g.ldb % 1024 ? 384 : 0);
+}
+
 // Past one round of the CUs, an aligned product whose K is no multiple of 64 (or whose rows of B are whole dwords only) has
 // the register-staged tiles (k_gemm_tiled) as the other choice: they start late, read far less a 64-deep step and win where K
 // is deep. Both as fitted to what they measured (us; k in 1024s, kn and nk the two layouts of B):

@@ -113,6 +113,7 @@ struct WavesPlan {
 constexpr int64_t kWavesMaxPartials = int64_t(12) << 20;
 bool waves_ok(const GemmArgs &g);
 WavesPlan waves_plan(const GemmArgs &g);
+bool waves_few_rows(const GemmArgs &g);       // whether it beats the few-rows kernels on rows they take (gemv_tiles_ok)
 bool staged_tile_faster(const GemmArgs &g);   // than its tiles past one round, of a product that tiled_fast_ok takes
 uint32_t waves_range_groups(const GemmArgs &g, const WavesPlan &p);   // its workgroups before slicing: one pair each
 int64_t waves_count(const GemmArgs &g, const WavesPlan &p);             // their waves

@@ -142,13 +142,14 @@ def test_float_and_requantized_forms_are_bit_exact(config):
 
 # Shapes that reach every kernel, each in some configuration (EVERY_KERNEL): few rows on the tiled few-rows kernels (or
 # split k), the waves kernel, the 128 and 256 direct kernels (ragged M included), the register-staged 128 tile (K = 96),
-# the generic kernel (unaligned rows), tiny products. The last three reach the one-launch few-rows kernel with its
+# the generic kernel (unaligned rows), tiny products. The last five reach the one-launch few-rows kernel with its
 # k-slices handed to the finishing tile (16 to 36 column slabs of 8 to 9 row bands), so its epilogues are checked after
-# a real hand-off.
+# a real hand-off, also with no spare row (16).
 REQUANT_KERNEL_SHAPES = [(1, 1, 1), (5, 7, 9), (4, 272, 512), (16, 256, 1024), (64, 64, 96), (33, 257, 77),
                          (128, 384, 384), (130, 256, 512), (2, 8192, 128), (96, 208, 320), (3, 4608, 272),
-                         (3, 4608, 1024), (16, 2048, 2048), (3, 4608, 4096), (4, 2048, 4096), (1, 2176, 4112)]
-HANDOFF_SHAPES = REQUANT_KERNEL_SHAPES[-3:]
+                         (3, 4608, 1024), (16, 2048, 2048), (3, 4608, 4096), (4, 2048, 4096), (1, 2176, 4112), (16, 2048, 4096),
+                         (5, 3072, 4096)]
+HANDOFF_SHAPES = REQUANT_KERNEL_SHAPES[-5:]
 EVERY_KERNEL = {
     "default": {"mfma-i8-rows16-xcd", "mfma-i8-rows16-direct", "mfma-i8-waves16x16x4", "mfma-i8-waves32x32x2"},
     "portable": {"portable-tile64x64x16"},
@@ -599,7 +600,7 @@ def test_few_rows_kernels_are_bit_exact(config):
             elif tiled and (one_launch or config == "tiles two launches"):
                 assert kernel == ("mfma-i8-rows16-xcd" if one_launch else "mfma-i8-rows16-tiles"), kernel
             else:   # too few slabs to hand over, or rows off 16 bytes
-                assert kernel.startswith(("mfma-i8-waves", "mfma-i8-rows16-direct")), kernel
+                assert kernel.startswith(("mfma-i8-waves", "mfma-i8-rows16-direct", "mfma-i8-rows16-tiles")), kernel
             bad_total += bad
     for vec in (False, True):
         say(f"{config} float vec {vec}")

@@ -30,6 +30,7 @@ CASES = [
     ("split k, ragged", 200, 144, 1536, 1, {"Tile": 64}, "mfma-i8-direct128x128x64-splitk", True),
     ("split k, as chosen", 150, 1408, 5120, 1, {}, "mfma-i8-direct128x128x64-splitk", True),
     ("few rows, one launch", 4, 2048, 4096, 1, {}, "mfma-i8-rows16-xcd", True),
+    ("few rows, one launch, 16 rows", 16, 2048, 4096, 1, {}, "mfma-i8-rows16-xcd", True),
     ("waves, 16 rows", 16, 4608, 1024, 1, {}, "mfma-i8-waves16x32x4", True),
     ("waves, batch 3", 128, 256, 320, 3, {}, "mfma-i8-waves32x32x2", True),
     ("waves, ragged", 200, 144, 192, 1, {}, "mfma-i8-waves32x32x2", True),
