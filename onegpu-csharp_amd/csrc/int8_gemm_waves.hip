@@ -564,6 +564,30 @@ bool waves_ok(const GemmArgs &g)
     return (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * g.batch <= (lim >> 5);
 }
 
+// Whether the 128 tile's split form is the faster for a walk of `steps` on t tiles: it cuts K finer than this kernel does.
+//  - Not sliced here, 80 steps and more (150 x 3456 x 5504 15.9 us there against 18.4, 32 x 8192 x 5120 14.5 against 16.7; 300 x 2048 x
+//    4672 15.4 against 18.4); from 60 with B stored N x K and CUs to spare (150 x 3456 x 4096 16.1 against 18.8, 46 x 4261 x 4608 14.2
+//    against 16.2, x 3584 equal; on 256 workgroups 64 x 4096 x 4672 14.4 against 9.3), from 70 where a fifth of the 64 x 64 tiles' rows is
+//    padding (96 x 8192 x 4608 18.9 against 22.1, x 4096 22.7 against 20.4). 5 to 16 rows of B stored N x K: 200 (16 x 1024 x 14336 13 against 16 to 17.5, x 8192 12 against 11).
+//  - B stored K x N, where the 128 tile splits: a step reads pieces of 64 rows, which HBM answers late. The line is where the mean of B
+//    from HBM and from the Infinity Cache is equal: on two waves 44 steps up to 32 rows (17 x 4096 x 3072 from HBM 11 against 15 us,
+//    from the cache 11 against 10; x 4096 13, 19 and 11, 12), 56 up to 64 (64 x 3072 x 4096 15, 20 and 14, 13), past that 60 on few
+//    tiles (96 x 1024 x 4096 13, 19 and 12, 10); 72 on larger tiles (64 x 5120 x 4608 19, 22 and 16, 16; 128 x 5120 x 4608 22, 26).
+//  - Sliced here: the slices are at most 8 to 16, there up to 64, which tells from 160 steps on wide results and from 200 on narrower
+//    ones (64 x 4096 x 11008 17 to 21.6 against 19 to 23.4; 96 x 2048 x 14336 N x K 17 against 21; but 64 x 512 x 11008 N x K 15 against 10).
+bool waves_walk_too_deep(const GemmArgs &g, int shape, int64_t t, int64_t steps, int64_t slices)
+{
+    const bool nk = g.flags & OG_GEMM_TRANSPOSE_B;
+    const int64_t cols = (int64_t)g.N * g.batch;
+    if (g.M <= 16) return nk && g.M > 4 && slices == 1 && steps >= 200;
+    if (slices > 1) return (!nk || g.M > 32) && (steps >= 200 ? cols >= 1536 : steps >= 160 && cols >= 3072);
+    if (steps >= 80) return true;
+    if (nk) return t <= 192 ? steps >= 60 : steps >= 70 && shape == S64x64W4 && (g.M + 63) / 64 * 256 > g.M * 5;
+    const int64_t most = shape == S32x32W2 ? (g.M <= 32 ? 44 : g.M <= 64 ? 56 : t <= 100 ? 60 : 80)
+                         : shape == S64x64W4 || (shape == S32x64W4 && g.M <= 64) ? 72 : 80;
+    return steps >= most && direct_split(g) > 1;
+}
+
 // The tile, waves and slices of K, from what sweeps of both layouts measured (MI355X, three sets of operands in turn):
 //  - The smallest tile whose workgroups still go round the chip's 256 CUs once is the fastest: its workgroups read
 //    the least each. 128 x 384 x 384: 32 x 32 (48 workgroups) 4.2 us, 32 x 64 5.2, 64 x 64 6.2; 512 x 768 x 3072: 32 x 64
@@ -571,10 +595,8 @@ bool waves_ok(const GemmArgs &g)
 //    A depth of 80 steps and more takes a larger tile for that, in slices that fill the round: 128 x 1024 x 8192 32 x 64 in
 //    four 12.3 us, 32 x 32 whole 22.6; 2 x 96 x 900 x 9856 64 x 64 in four 16.8, 32 x 32 whole 49.
 //  - Against the 128 tile fed by LDS DMA, one whole round of 64 x 64 also needs 16 steps to win (1024 x 1024 x 4096
-//    21.4 -> 17.3 us, 256 x 4096 x 1024 8.8 -> 8.4, 1024 x 768 x 768 equal; 512 x 1536 x 384 6.5 -> 6.8). A deep K that is not
-//    sliced here is sliced there, which wins from 80 steps on (150 x 3456 x 5504 15.9 us against 18.4, 32 x 8192 x 5120 14.5 against 16.7;
-//    300 x 2048 x 4672 18.4 against 15.4), from 60 with B stored N x K and CUs to spare (150 x 3456 x 4096 16.1 against 18.8, 46 x 4261 x
-//    4608 14.2 against 16.2, x 3584 equal; on 256 workgroups 64 x 4096 x 4672 14.4 against 9.3).
+//    21.4 -> 17.3 us, 256 x 4096 x 1024 8.8 -> 8.4, 1024 x 768 x 768 equal; 512 x 1536 x 384 6.5 -> 6.8). A deep K goes to its split
+//    form (waves_walk_too_deep).
 //  - With more than one round (one_round false), the largest tile on one or two waves, so that several workgroups
 //    share a CU: 2000 x 2001 x 2003: 64 x 64 on two waves 54 us, on four 60; 333 x 64 x 333 x 96: 32 x 64 on one wave 12.4 us, 64 x 64
 //    on two 13.5; 1 x 51865 x 768: 16 x 64 on one wave 10.3 us, on four 12.9.
@@ -624,8 +646,7 @@ WavesPlan waves_plan(const GemmArgs &g)
     // The slices' int32 sums stay within what every context's workspace and the fixed scratch hold from the start.
     slices = std::min<int64_t>(slices, kWavesMaxPartials / std::max<int64_t>((int64_t)g.M * g.N * g.batch * 4, 1));
     slices = std::max<int64_t>(slices, 1);
-    const int64_t deepest = trans_b && t <= 192 ? 60 : 80;
-    p.beats_direct = p.one_round && !(slices == 1 && ((p.shape == S64x64W4 && steps < 16) || (g.M > 16 && steps >= deepest)));
+    p.beats_direct = p.one_round && !(slices == 1 && p.shape == S64x64W4 && steps < 16) && !waves_walk_too_deep(g, p.shape, t, steps, slices);
     p.slice_steps = (int32_t)((steps + slices - 1) / slices);
     p.slices = (int32_t)((steps + p.slice_steps - 1) / p.slice_steps);
     return p;

@@ -586,6 +586,17 @@ def test_kernel_choice_is_reported():
     # A K of 80 steps and more over more tiles than it can be sliced for goes back to the split 128 tile.
     assert name(M=150, N=1408, K=5120) == "mfma-i8-direct128x128x64-splitk"
     assert name(M=128, N=1024, K=8192) == "mfma-i8-waves32x64x4-splitk"
+    # Walks too deep for one tile's waves: on two waves by the rows and the tiles, larger tiles, rows that are padding, slices
+    # of K; where the 128 tile does not split, the waves keep the product.
+    split = "mfma-i8-direct128x128x64-splitk"
+    assert name(M=17, N=4096, K=2752) == "mfma-i8-waves32x32x2" and name(M=17, N=4096, K=2816) == split
+    assert name(M=64, N=3072, K=3520) == "mfma-i8-waves32x32x2" and name(M=64, N=3072, K=3584) == split
+    assert name(M=96, N=1024, K=3776) == "mfma-i8-waves32x32x2" and name(M=96, N=1024, K=3840) == split
+    assert name(M=96, N=2048, K=4096) == "mfma-i8-waves32x32x2" and name(M=128, N=3072, K=4096) == "mfma-i8-waves32x64x4"
+    assert name(M=64, N=5120, K=4544) == "mfma-i8-waves32x64x4" and name(M=64, N=5120, K=4608) == split
+    assert name(M=96, N=8192, K=4096, Flags=0x4) == "mfma-i8-waves64x64x4" and name(M=96, N=8192, K=4608, Flags=0x4) == split
+    assert name(M=64, N=4096, K=8192) == "mfma-i8-waves64x64x4-splitk" and name(M=64, N=4096, K=11008) == split
+    assert name(M=64, N=512, K=11008) == "mfma-i8-waves32x32x4-splitk" and name(M=16, N=1024, K=14336, Flags=0x4) == split
     # Aligned, K no multiple of 64, past one round: the register-staged tiles where K is deep, both layouts of B, a B whose
     # rows are whole dwords only, a tall result, and one round of them alone.
     for k, want in ((400, "mfma-i8-waves64x64x2"), (4080, "mfma-i8-tile256x256x64")):
