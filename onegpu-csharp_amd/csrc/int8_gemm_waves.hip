@@ -702,11 +702,11 @@ bool staged_tile_faster(const GemmArgs &g)
     return staged < waves;
 }
 
-int64_t waves_count(const GemmArgs &g, const WavesPlan &p)
-{
-    static const int waves[] = {4, 4, 4, 1, 4, 2, 4, 4, 1, 4, 2};
-    return (int64_t)waves_range_groups(g, p) * waves[p.shape];
-}
+constexpr int kShapeWaves[] = {4, 4, 4, 1, 4, 2, 4, 4, 1, 4, 2};
+
+int64_t waves_count(const GemmArgs &g, const WavesPlan &p) { return (int64_t)waves_range_groups(g, p) * kShapeWaves[p.shape]; }
+
+double waves_walk(const WavesPlan &p) { return (double)p.slice_steps / kShapeWaves[p.shape]; }
 
 uint32_t waves_range_groups(const GemmArgs &g, const WavesPlan &p)
 {

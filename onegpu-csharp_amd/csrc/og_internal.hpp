@@ -117,6 +117,7 @@ bool waves_few_rows(const GemmArgs &g);       // whether it beats the few-rows k
 bool staged_tile_faster(const GemmArgs &g);   // than its tiles past one round, of a product that tiled_fast_ok takes
 uint32_t waves_range_groups(const GemmArgs &g, const WavesPlan &p);   // its workgroups before slicing: one pair each
 int64_t waves_count(const GemmArgs &g, const WavesPlan &p);             // their waves
+double waves_walk(const WavesPlan &p);                                  // 64-deep steps a wave takes
 // A convolution's column matrix as that kernel reads it straight from the images (g.B the first image's channels of
 // the group, g.strideB the bytes of an image, g.K = channels * taps, g.N the output's positions, g.ZB what the padding
 // holds): unit strides, output rows as long as the input's, at most kConvMaxTaps taps, K below 2^25.

@@ -23,12 +23,16 @@ GEOMETRIES = [
     (2, 11, 16, 16, 24, 3, 3, (2, 2, 2, 2), (2, 2), 1),      # dilation
     (1, 6, 12, 33, 50, 4, 2, (1, 0, 2, 1), (1, 1), 1),       # even windows
     (1, 80, 1, 333, 70, 1, 3, (0, 1, 0, 1), (1, 1), 1),      # one dimension
-    (2, 12, 9, 10, 16, 3, 3, (1, 1, 1, 1), (1, 1), 2),       # groups
+    (4, 40, 31, 31, 34, 3, 3, (1, 1, 1, 1), (1, 1), 2),      # groups
     (1, 40, 10, 10, 5, 7, 7, (3, 3, 3, 3), (1, 1), 1),       # 49 taps, few rows
     (1, 600, 8, 8, 40, 3, 3, (1, 1, 1, 1), (1, 1), 1),       # slices of K (5400)
     (8, 10, 50, 50, 96, 3, 3, (1, 1, 1, 1), (1, 1), 1),      # more tiles than CUs
     (4, 37, 7, 9, 65, 1, 1, (0, 0, 0, 0), (1, 1), 1),        # 1 x 1 over rows of 63 bytes
-    (30, 20, 31, 31, 100, 1, 1, (0, 0, 0, 0), (1, 1), 1)]    # 1 x 1, more tiles than CUs
+    (30, 20, 31, 31, 100, 1, 1, (0, 0, 0, 0), (1, 1), 1),    # 1 x 1, more tiles than CUs
+    (2, 12, 9, 10, 16, 3, 3, (1, 1, 1, 1), (1, 1), 2),       # packed: two groups of a small matrix, many groups, a long
+    (1, 48, 14, 14, 96, 3, 3, (1, 1, 1, 1), (1, 1), 12),     # walk on two waves
+    (1, 512, 14, 14, 512, 3, 3, (1, 1, 1, 1), (1, 1), 1)]
+PACKED = GEOMETRIES[-3:]
 
 
 @pytest.mark.parametrize("index", range(len(GEOMETRIES)))
@@ -45,4 +49,4 @@ def test_convolutions_without_a_column_matrix_are_bit_exact(index):
         say(f"{c['name']} pads {pads} dilation {dil} groups {groups} signed {c['xs']}/{c['ws']} zp {c['xzm']}/{c['wzm']}")
         bad, kern = _run_case(d, conv, c, 7000 + 10 * index + s)
         assert bad == 0, f"{c['name']}: {bad} elements differ ({kern})"
-        assert kern.startswith("conv-waves" if kh * kw > 1 else "mfma-i8-waves"), kern
+        assert kern.startswith("conv-waves") == (kh * kw > 1 and GEOMETRIES[index] not in PACKED), kern
