@@ -553,7 +553,9 @@ void launch_waves_as(const GemmArgs &g, int32_t ksplit, int32_t slice_steps, con
 
 }  // namespace
 
-// Conditions of the kernel: rows of at least one 16-byte piece, every offset of a tile's buffer under 2^31.
+// Conditions of the kernel: rows of at least one 16-byte piece, every offset of a tile's buffer under 2^31, and fewer than
+// 2^32 threads in the grid, which is what a launch takes (a batch of millions of narrow products passes that on four waves
+// a tile).
 bool waves_ok(const GemmArgs &g)
 {
     const bool trans_b = g.flags & OG_GEMM_TRANSPOSE_B;
@@ -561,7 +563,8 @@ bool waves_ok(const GemmArgs &g)
     if (g.M < 1 || g.N < 1 || g.K < 16 || (!trans_b && g.N < 16)) return false;
     if ((int64_t)63 * g.lda + g.K > lim) return false;
     if (trans_b ? (int64_t)127 * g.ldb + g.K > lim : (int64_t)(g.K + 63) * g.ldb > lim) return false;
-    return (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * g.batch <= (lim >> 5);
+    if ((int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * g.batch > (lim >> 5)) return false;
+    return (waves_count(g, waves_plan(g)) + 64) * 64 < (1ll << 32);
 }
 
 // Whether the 128 tile's split form is the faster for a walk of `steps` on t tiles: it cuts K finer than this kernel does.

@@ -541,6 +541,10 @@ def test_kernel_choice_is_reported():
         lib.og_int8_gemm_kernel_name(ctypes.byref(GemmParams(**kw)), 1, out, 64)
         return out.value.decode()
 
+    def many(k, n, batch, flags=0):
+        lib.og_int8_gemm_kernel_name(ctypes.byref(GemmParams(M=1, N=n, K=k, Flags=flags)), batch, out, 64)
+        return out.value.decode()
+
     def tiled(**kw):   # OG_GEMM_NO_SKINNY: the tiled kernels, whatever the size
         return name(**{**kw, "Flags": kw.get("Flags", 0) | 0x800})
 
@@ -606,6 +610,9 @@ def test_kernel_choice_is_reported():
     assert name(M=2000, N=1504, K=3088) == name(M=300, N=4096, K=2000, Flags=0x4) == "mfma-i8-waves64x64x2"
     assert name(M=300, N=4096, K=2000) != name(M=128, N=50304, K=4112, Flags=0x4) == "mfma-i8-tile128x128x128"
     assert name(M=4096, N=4097, K=4099) == "mfma-i8-waves64x64x2"             # unaligned: only the generic kernel is left
+    # A launch takes fewer than 2^32 threads: four waves a tile for a batch of at most 2^24 - 1 tiles.
+    assert many(16, 17, 2**23) == "mfma-i8-rows16-direct" and many(16, 17, 2**22) == "mfma-i8-waves16x16x4"
+    assert many(16, 17, 2**23, 0x4) == "mfma-i8-waves16x64x1"
     # Tiles of 256 that are mostly padding, or partial ones with byte sums of A, are left for 128.
     def wide(m, n, k, batch, flags=0x2):
         lib.og_int8_gemm_kernel_name(ctypes.byref(GemmParams(M=m, N=n, K=k, Flags=flags, StrideA=m * k, StrideB=k * n)), batch, out, 64)

@@ -8,6 +8,7 @@ block, so they are cheap to make; the extreme values of x sit at its first and l
 last workgroup."""
 from __future__ import annotations
 
+import ctypes
 import gc
 
 import numpy as np
@@ -15,7 +16,7 @@ import pytest
 
 import oracle
 import onegpu_hip as og
-from gpu_rig import device, run, say
+from gpu_rig import abi, binding, check, device, run, say
 
 pytestmark = pytest.mark.gpu
 
@@ -144,3 +145,22 @@ def test_gather_from_a_table_past_4_gib():
     bad = int(np.count_nonzero(got != want))
     say(f"ROW gather past 4 GiB | {kernel} | mismatching elements {bad}")
     assert bad == 0
+
+
+def test_a_batch_of_millions_of_narrow_products():
+    # 2^23 products of 1 x 17 x 16 that share A and B: on four waves a tile the launch would have 2^32 threads, one more
+    # than it takes, so another kernel runs. Every row of C is the same.
+    d, L = device(), abi()
+    batch, n, k = 2**23, 17, 16
+    rng = np.random.default_rng(3)
+    a, b = rng.integers(0, 256, k, dtype=np.uint8), rng.integers(-128, 128, k * n, dtype=np.int8)
+    want = oracle.int8_gemm(oracle.Gemm(1, n, k), a, False, b.view(np.uint8), True)
+    ba, bb, bc = d.CreateBuffer(a), d.CreateBuffer(b), d.CreateBufferOf(og.ElementType.Int32, batch * n)
+    prm = L.GemmParams(M=1, N=n, K=k, Lda=k, Ldb=n, Flags=0x2, StrideC=n)
+    none = L.Buf(None, 0)
+    say(f"{batch} products of 1 x {n} x {k}")
+    check(L.og_int8_gemm(d.Context, ctypes.byref(prm), batch, binding(ba), binding(bb), binding(bc), none, none, none,
+                         none, none), d)
+    d.WaitIdle()
+    assert d.LastKernel == "mfma-i8-rows16-direct", d.LastKernel
+    assert np.all(bc.Read().reshape(batch, n) == want)
