@@ -145,8 +145,8 @@ __device__ __forceinline__ void waves_tile(const GemmArgs &g, const ConvView &cv
     const bool a_signed = g.flags & OG_GEMM_A_INT8, b_signed = g.flags & OG_GEMM_B_INT8;
     const int32_t flip_a = a_signed ? 0 : (int32_t)0x80808080, flip_b = b_signed ? 0 : (int32_t)0x80808080;
 
-    // The tile's operand ranges, from a whole dword (MIS: to a whole dword; what a dword holds past the operand is
-    // never used).
+    // The tile's operand ranges (MIS: from and to a whole dword; what a dword holds past the operand is never used, and
+    // lies inside the operand's buffer, GEMM_WHOLE_DWORDS).
     const uint8_t *const a_at = g.A + batch * g.strideA + (int64_t)m0 * lda;
     const uint8_t *const b_at = g.B + batch * g.strideB + (CONV ? (int64_t)0 : TRANS_B ? (int64_t)n0 * ldb : (int64_t)n0);
     const uint32_t a_skip = MIS ? (uint32_t)(uintptr_t)a_at & 3u : 0u, b_skip = MIS ? (uint32_t)(uintptr_t)b_at & 3u : 0u;
@@ -555,11 +555,12 @@ void launch_waves_as(const GemmArgs &g, int32_t ksplit, int32_t slice_steps, con
 
 // Conditions of the kernel: rows of at least one 16-byte piece, every offset of a tile's buffer under 2^31, and fewer than
 // 2^32 threads in the grid, which is what a launch takes (a batch of millions of narrow products passes that on four waves
-// a tile).
+// a tile). The form for N x K operands off a dword reads whole dwords, which must lie inside the operands' buffers.
 bool waves_ok(const GemmArgs &g)
 {
     const bool trans_b = g.flags & OG_GEMM_TRANSPOSE_B;
     const int64_t lim = 0x7FFFFFFFll - 512;
+    if (trans_b && waves_off_dword(g) && !(g.flags & GEMM_WHOLE_DWORDS)) return false;
     if (g.M < 1 || g.N < 1 || g.K < 16 || (!trans_b && g.N < 16)) return false;
     if ((int64_t)63 * g.lda + g.K > lim) return false;
     if (trans_b ? (int64_t)127 * g.ldb + g.K > lim : (int64_t)(g.K + 63) * g.ldb > lim) return false;

@@ -40,6 +40,10 @@ struct GemmArgs {
 // Pairs a ranged product may write: its caller's buffer holds 2 * kRangesMax floats (OG_RANGES_MAX).
 constexpr int kRangesMax = 1024;
 
+// Library-internal bit of GemmArgs::flags (above the public OG_GEMM_* ones): the whole dwords that hold the first and last
+// bytes of A and of B lie inside their buffers.
+constexpr uint32_t GEMM_WHOLE_DWORDS = 0x10000u;
+
 // Library-internal epilogue bits (above the public OG_EPI_* ones): C is 8-bit and each sum is requantized with the
 // multiplier at `scale` and the zero point zp_y; uint8 output when EPI_REQUANT_U8, else int8.
 constexpr uint32_t EPI_REQUANT = 0x100u, EPI_REQUANT_U8 = 0x200u;

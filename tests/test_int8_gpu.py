@@ -462,6 +462,33 @@ def test_b_ending_at_its_last_valid_byte_takes_another_kernel():
         assert np.array_equal(bc.Read(), want)
 
 
+def test_operands_off_a_dword_are_read_inside_their_buffers():
+    # B stored N x K, rows off a dword: the waves kernel reads whole dwords of A and B there. With a buffer that starts or
+    # ends inside such a dword (through the C ABI; the host layer's buffers are whole words) the byte-exact kernel runs, with
+    # the same sums.
+    d, L = device(), abi()
+    m, n, k = 33, 47, 201
+    rng = np.random.default_rng(6)
+    a, b = rng.integers(0, 256, m * k + 8, dtype=np.uint8), rng.integers(0, 256, n * k + 8, dtype=np.uint8)
+    ba, bb, bc = d.CreateBuffer(a), d.CreateBuffer(b), d.CreateBufferOf(og.ElementType.Int32, m * n)
+    none = L.Buf(None, 0)
+    whole, exact = "mfma-i8-waves32x32x2", "mfma-i8-generic128x128x64"
+    # For A and B: where the buffer starts, the operand's offset in it, the bytes past its end.
+    for at_a, off_a, past_a, at_b, off_b, past_b, want_kernel in (
+            (0, 1, 4, 0, 3, 4, whole), (1, 0, 4, 0, 3, 4, exact), (0, 1, 4, 3, 0, 4, exact), (0, 3, 0, 0, 3, 4, whole),
+            (0, 2, 0, 0, 3, 4, exact), (0, 2, 1, 0, 3, 4, whole), (0, 1, 4, 0, 1, 0, whole), (0, 1, 4, 0, 2, 0, exact)):
+        sa, sb = at_a + off_a, at_b + off_b
+        want = oracle.int8_gemm(oracle.Gemm(m, n, k, TransposeB=1), a[sa:sa + m * k], False, b[sb:sb + n * k], False)
+        say(f"A from {at_a} + {off_a}, {past_a} past; B from {at_b} + {off_b}, {past_b} past")
+        prm = L.GemmParams(M=m, N=n, K=k, Lda=k, Ldb=k, OffA=off_a, OffB=off_b, Flags=0x4, StrideC=m * n)
+        check(L.og_int8_gemm(d.Context, ctypes.byref(prm), 1, L.Buf(ba.DevicePointer + at_a, off_a + m * k + past_a),
+                             L.Buf(bb.DevicePointer + at_b, off_b + n * k + past_b), binding(bc), none, none, none, none,
+                             none), d)
+        d.WaitIdle()
+        assert d.LastKernel == want_kernel, d.LastKernel
+        assert np.array_equal(bc.Read(), want)
+
+
 # Products split along K on the 128 x 128 direct kernel: its grid fills under half the chip, and K has at least 8 stages.
 # The first five ask for the tiled kernels; the others come there by themselves: a deep K over more tiles than the waves
 # kernel cuts into slices.
