@@ -156,8 +156,9 @@ int og_int8_gemm(og_ctx *ctx, const og_int8_gemm_params *params, uint32_t batch,
                  og_buffer ZA, og_buffer ZB, og_buffer bias, og_buffer scale, og_buffer fbias);
 
 /* og_int8_gemm that allocates nothing: no counterpart in the reference. For callers that cannot allocate device
- * memory (work captured into a HIP graph, serving loops, harnesses that forbid hipMalloc). The same product, kernels
- * and result; the scratch its kernels need (split-k and few-rows partial sums, the few-rows kernel's count words)
+ * memory (work captured into a HIP graph, serving loops, harnesses that forbid hipMalloc). The same product
+ * and result (and kernel, but few-rows products of 16 column slabs of 128 and more all run in one launch,
+ * "mfma-i8-rows16-xcd"); the scratch its kernels need (split-k and few-rows partial sums, the few-rows kernel's count words)
  * comes from one fixed array of OG_NOALLOC_SCRATCH_BYTES per device instead of the context's workspace. A product
  * that needs more fails with OG_ERR_UNSUPPORTED before anything is launched. Every call on a device shares that
  * device's array (whatever the context), so calls that overlap on one device race. */

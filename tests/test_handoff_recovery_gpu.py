@@ -17,7 +17,7 @@ import pytest
 
 import oracle
 import onegpu_hip as og
-from gpu_rig import abi, binding, say
+from gpu_rig import abi, binding, run, say
 
 pytestmark = pytest.mark.gpu
 
@@ -101,6 +101,23 @@ def test_give_up_reported_words_cleared_two_launch_form_after():
         assert pr.launch() == (0, "mfma-i8-rows16-tiles")
         assert pr.sync() == 0 and pr.bit_exact()
     del pr, d
+
+
+def test_the_spin_limit_chooses_no_kernel():
+    # The hook changes how long a finishing tile waits, not which kernel a product runs on.
+    L = _lib()
+    d = og.GpuDevice.Create(0)
+    gemm, kernels = og.Int8Gemm(d), []
+    for limit in (1 << 22, (1 << 22) - 1):
+        assert L.og_test_set_spin_limit(d.Context, limit) == 0
+        for m, n, k in ((16, 2048, 1024), (4, 8192, 2048), (4, 2048, 4096)):
+            a, b = d.CreateBuffer(np.ones(m * k, np.uint8)), d.CreateBuffer(np.ones(k * n, np.int8))
+            c = d.CreateBufferOf(og.ElementType.Int32, m * n)
+            say(f"spin limit {limit}: {m}x{n}x{k}")
+            run(d, lambda e: gemm.EncodeInt32(e, og.Int8GemmProblem(m, n, k), a, b, c))
+            kernels.append(d.LastKernel)
+            assert np.all(c.Read() == k)
+    assert kernels[:3] == kernels[3:], kernels
 
 
 def test_poisoned_fixed_words_are_reported_by_another_context():
