@@ -13,8 +13,8 @@
 // (w - wz) (xz - xz) = 0, and the same launch copies the weights into rows of kp bytes, zero past k; the 16-byte
 // chunks of both go through one grid-stride loop (the column chunks first).
 //
-// Depthwise (one input channel a group): no matrix at all. The usual windows go by tiles through LDS
-// (k_conv_depthwise_tile); any other one has a thread per output element, which sums its KH * KW taps,
+// Depthwise (one input channel a group): no matrix at all. The usual windows over enough outputs go by tiles through LDS
+// (k_conv_depthwise_tile); any other convolution has a thread per output element, which sums its KH * KW taps,
 // (x - xz) * (w - wz[m]) in 32-bit wrap-around, skipping taps in the padding (they are the real value zero).
 #include "og_internal.hpp"
 
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv_depthwise(ConvDepthwiseAr
 // A tile is `c` planes (whole ones, or a part of one) of `trg` groups of R rows of `tcq` quads of columns.
 // Bound by memory at the large end: 8 x 512 channels of 112 x 112, 5 x 5, 770 -> 92 us (205 MB of results and 51 MB of input
 // are 50 us at the rate of a large copy), 3 x 3 299 -> 66, with strides of 2 90 -> 36; 2 x 64 of 223 x 223, 5 x 5 by 2, 34.0 -> 8.7;
-// one dimension, 8 x 512 of 2999, 5 taps, 69.6 -> 26.9; by the launch at the small one: 256 x 14 x 14, 8 images, 4.9 -> 4.7, 16 x 7 x 7 4.0.
+// one dimension, 8 x 512 of 2999, 5 taps, 69.6 -> 26.9. Small ones are bound by the launch and by staging (depthwise_by_output).
 struct DepthwiseTile {
     int32_t tcq, trg, c, coltiles, rowtiles, rows_in, stride, planes, cout_g;   // stride: words of a staged row
     uint32_t magic_stride, magic_rows;                                          // as ConvView's
@@ -351,11 +351,26 @@ hipError_t launch_depthwise_tile(const ConvDepthwiseArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+// Whether a thread per output is the faster, by what both kernels measured over 64 to 16384 planes of 1 to 12544 outputs (us,
+// thread per output against tile):
+//  - 3 x 3, staging costs more than 18 byte loads until there are some 180000 outputs: 1024 x 10 x 10 3.6, 4.0; 1024 x 14 x 14 4.4, 4.1;
+//    4096 x 14 x 14 8.4, 5.6; on planes of under 16 outputs at any number: 16384 x 3 x 3 4.0, 5.2. With strides of 2, which stage four
+//    times the outputs, the planes must be larger: 4096 x 10 x 10 5.9, 6.5; 16384 x 10 x 10 13.3, 12.4; 1024 x 20 x 20 5.8, 5.3;
+//  - 5 x 5, 50 byte loads, the tile wins on all but the smallest planes: 1024 x 3 x 3 5.5, 4.1; 4096 x 2 x 2 3.9, 5.1;
+//  - one dimension: 256 x 300 3.3, 3.2; 1024 x 300 4.4, 3.8; 64 x 300 2.9, 3.2.
+bool depthwise_by_output(const ConvDepthwiseArgs &a, int64_t results)
+{
+    const int64_t plane = (int64_t)a.oh * a.ow;
+    if (a.kh == 1) return results < (a.sw == 1 ? 75000 : 150000);
+    if (a.kh == 3) return a.sw == 1 ? results < 180000 || plane < 16 : results < (plane < 400 ? 800000 : 180000) || plane < 100;
+    return plane < 9 && !(a.sw == 2 && plane >= 4 && results <= 4096 * plane);
+}
+
 // Whether k_conv_depthwise_tile covers the window; the extents and the results' number keep its 32-bit positions and grid.
 bool depthwise_tile_ok(const ConvDepthwiseArgs &a, int64_t results)
 {
     constexpr int32_t limit = 1 << 28;
-    return results < (1 << 30) && a.dh == 1 && a.dw == 1 && (a.kw == 3 || a.kw == 5) && (a.kh == a.kw || a.kh == 1) && (a.sw == 1 || a.sw == 2) &&
+    return !depthwise_by_output(a, results) && results < (1 << 30) && a.dh == 1 && a.dw == 1 && (a.kw == 3 || a.kw == 5) && (a.kh == a.kw || a.kh == 1) && (a.sw == 1 || a.sw == 2) &&
            (a.sh == a.sw || (a.kh == 1 && a.oh == 1)) && a.h < limit && a.w < limit && a.oh < limit && a.ow < limit &&
            a.ph < limit && a.pw < limit;
 }
@@ -384,6 +399,7 @@ hipError_t launch_conv_depthwise(const ConvDepthwiseArgs &a, hipStream_t s, cons
     const int64_t total = (int64_t)a.batch * a.cout * a.oh * a.ow;
     if (total == 0) return hipSuccess;
     if (depthwise_tile_ok(a, total)) {
+        *kernel = "conv-depthwise-tile-i8";
         const bool one = a.sw == 1;
         if (a.kh == 3) return one ? launch_depthwise_tile<3, 3, 1, 4>(a, s) : launch_depthwise_tile<3, 3, 2, 4>(a, s);
         if (a.kh == 5) return one ? launch_depthwise_tile<5, 5, 1, 4>(a, s) : launch_depthwise_tile<5, 5, 2, 4>(a, s);
