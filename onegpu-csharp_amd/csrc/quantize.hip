@@ -47,9 +47,20 @@ __device__ void dq_params(float mn, float mx, float &scale, uint32_t &zp)
 }
 
 // Pass 1: each workgroup's range (NaN-ignoring min and max) over its grid-stride share of x. Bound by memory. Its loads are
-// plain ones, so that what fits the 4 MiB of each XCD's L2 is there for pass 2, whose workgroups read the same 16 KiB
-// blocks from the same XCDs: 1.9 M elements dequantized and quantized 16.0 -> 15.7 us, 6.9 M 26.6 -> 25.6 against
-// non-temporal loads, 12.6 M 36.8 -> 37.1.
+// plain ones (NT false), so that what fits the caches is there for pass 2, whose workgroups read the same 16 KiB blocks from
+// the same XCDs: 1.9 M elements dequantized and quantized 16.0 -> 15.7 us, 6.9 M 26.6 -> 25.6 against non-temporal loads; alone,
+// 12.6 M 22.0 -> 20.4, 33 M 52 -> 49. Past 160 MB of x its head is gone before pass 2 comes, and the plain loads only push out
+// what else was there: 50 M elements 69 -> 79, 67 M 93 -> 102, 200 M 284 -> 303, so those are non-temporal (42 M equal).
+constexpr uint32_t kDqPlainMax = 40u << 20;
+
+template <bool NT>
+__device__ __forceinline__ f4 dq_load(const f4 *p)
+{
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
+template <bool NT>
 __global__ __launch_bounds__(DQ1_THREADS) void k_dq_minmax(const float *x, uint32_t count, float *ranges)
 {
     __shared__ float red[2 * DQ1_THREADS / 64];
@@ -64,14 +75,14 @@ __global__ __launch_bounds__(DQ1_THREADS) void k_dq_minmax(const float *x, uint3
         for (; i + 3 * nthreads < n4; i += 4 * nthreads) {
             f4 v[4];
 #pragma unroll
-            for (int q = 0; q < 4; q++) v[q] = x4[i + q * nthreads];
+            for (int q = 0; q < 4; q++) v[q] = dq_load<NT>(&x4[i + q * nthreads]);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 minmax_acc(v[q].x, mn, mx); minmax_acc(v[q].y, mn, mx); minmax_acc(v[q].z, mn, mx); minmax_acc(v[q].w, mn, mx);
             }
         }
         for (; i < n4; i += nthreads) {
-            const f4 v = x4[i];
+            const f4 v = dq_load<NT>(&x4[i]);
             minmax_acc(v.x, mn, mx); minmax_acc(v.y, mn, mx); minmax_acc(v.z, mn, mx); minmax_acc(v.w, mn, mx);
         }
         for (uint32_t i = n4 * 4 + tid; i < count; i += nthreads) minmax_acc(x[i], mn, mx);
@@ -257,12 +268,18 @@ static uint32_t dq_groups(uint32_t count)
     return g < 1 ? 1 : (g > (uint32_t)kDqMaxGroups ? (uint32_t)kDqMaxGroups : g);
 }
 
+static void launch_dq_minmax(const float *x, uint32_t count, float *ranges, uint32_t groups, hipStream_t s)
+{
+    if (count > kDqPlainMax) hipLaunchKernelGGL(k_dq_minmax<true>, dim3(groups), dim3(DQ1_THREADS), 0, s, x, count, ranges);
+    else hipLaunchKernelGGL(k_dq_minmax<false>, dim3(groups), dim3(DQ1_THREADS), 0, s, x, count, ranges);
+}
+
 hipError_t launch_dynamic_quantize(const DqArgs &d, const Workspace &ws, hipStream_t s, const char **kernel, int step)
 {
     const uint32_t groups = dq_groups(d.count);
     if (step == 0) {
         *kernel = "dq-minmax";
-        hipLaunchKernelGGL(k_dq_minmax, dim3(groups), dim3(DQ1_THREADS), 0, s, d.x, d.count, ws.dq_ranges);
+        launch_dq_minmax(d.x, d.count, ws.dq_ranges, groups, s);
     } else {
         *kernel = "dq-quantize";
         // One block of 4096 elements a workgroup (at most 2^20 workgroups for a 32-bit count).
@@ -292,7 +309,7 @@ hipError_t launch_range_pass(const float *x, uint32_t count, float *ranges, hipS
 {
     *kernel = "dq-minmax";
     *groups = dq_groups(count);
-    hipLaunchKernelGGL(k_dq_minmax, dim3(*groups), dim3(DQ1_THREADS), 0, s, x, count, ranges);
+    launch_dq_minmax(x, count, ranges, *groups, s);
     return hipGetLastError();
 }
 
