@@ -27,15 +27,16 @@ bool direct_ok(const GemmArgs &g)
 //    256 tile pads more than that: 96 x 333 x 336 x 256 (512 x 512 against 384 x 384) 19.4 against 26.9 us, 64 x 128 x 3072 x 256 43.9
 //    against 54.7, 14 x 40 x 3712 x 1024 15.7 against 21.8;
 //  - with A's byte sums (B unsigned or with a zero point) the 256 tile stores partial tiles slowly, and wins only on
-//    whole ones (4096 x 4096 x 1024 32.6 against 35.8 us; but 4000 x 4000 x 1024 42.0 against 35.3, 96 x 333 x 336 x 64 41.7
-//    against 16.8) or where a deep K outweighs it (16 x 1000 x 1024 x 2048 52 against 65).
+//    whole ones (4096 x 4096 x 1024 32.6 against 35.8 us; but 4000 x 4000 x 1024 36.5 against 34.9, x 256 25.1 against 19.5, 96 x
+//    333 x 336 x 64 41.7 against 16.8) or where a deep K outweighs it: in one round of tiles past 1024 (3600 x 3600 x 1152 34.0 against
+//    37.4, 16 x 1000 x 1024 x 1536 48 against 58, x 2048 52 against 65), in more from 2048 (5000 x 5008 x 1280 69.6 against 66.3).
 bool direct_uses_large(const GemmArgs &g)
 {
     if (g.flags & OG_GEMM_LARGE_TILE) return true;
     if (!tiled_uses_large(g.M, g.N, g.batch)) return false;
     const bool sum_a = (g.flags & OG_GEMM_ZB) || !(g.flags & OG_GEMM_B_INT8);
-    if (sum_a && g.K < 2048) return g.M % 256 == 0 && g.N % 256 == 0;
     const int64_t area256 = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256) * 4;
+    if (sum_a && g.K < (area256 * g.batch <= 1024 ? 1152 : 2048)) return g.M % 256 == 0 && g.N % 256 == 0;
     const int64_t area128 = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
     return area256 * 100 <= area128 * (g.K <= 1024 || sum_a ? 115 : 175);
 }

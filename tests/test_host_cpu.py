@@ -619,6 +619,8 @@ def test_kernel_choice_is_reported():
         return out.value.decode()
 
     assert wide(40, 304, 64, 200) == wide(129, 272, 128, 104, 0x2 | 0x60) == "mfma-i8-direct128x128x64"
+    assert wide(3600, 3600, 1024, 1, 0) == wide(5000, 5008, 1536, 1, 0x22) == "mfma-i8-direct128x128x64"
+    assert wide(3600, 3600, 1152, 1, 0) == wide(5000, 5008, 2048, 1, 0x22) == "mfma-i8-direct256x256x64"
     assert wide(256, 256, 64, 200, 0) == wide(250, 512, 64, 101) == "mfma-i8-direct256x256x64"
 
 
