@@ -665,15 +665,16 @@ WavesPlan waves_plan(const GemmArgs &g)
 //   1 x 4096 x 1280     from HBM 7.2, 6.7    from the cache 6.9, 6.4      16 x 4096 x 4096    11.5, 13.8    10.9, 10.4
 //   1 x 4096 x 3584              8.8, 12.1             7.9, 9.2           16 x 11008 x 4096   16.7, 15.0    16.1, 11.0
 //   5 x 8192 x 4096              13, 16                 12, 11.5          16 x 3072 x 5120    12, 16        -
-// Past one round the walk is one wave's alone: 40960 columns of 3072, one row, 27 against 39 us; of 768, 13 against 13. A
-// depth of at most 512 is one part, with nothing to hand over: 1 x 28672 x 512 8.0 against 8.5.
+// Past one round the walk is one wave's alone: 40960 columns of 3072, one row, 27 against 39 us; of 1024, 16 against 16, from the
+// cache 15 against 12. A depth of at most 512 is one part, with nothing to hand over: 1 x 28672 x 512 8.0 against 8.5. Under 16 slabs
+// of columns the other choice is the two-launch form: 1 x 1024 x 1024 7.7 against 5.3, 8 x 1024 x 4096 8.1 against 11.6.
 bool waves_few_rows(const GemmArgs &g)
 {
     const int64_t cols = (int64_t)g.N * g.batch, slabs = (int64_t)((g.N + 127) / 128) * g.batch;
-    if (slabs < 16) return g.K <= 2560;   // the two-launch form: 1 x 1024 x 1024 7.7 against 5.3 us, 8 x 1024 x 4096 8.1 against 11.6 from HBM
+    if (slabs < 16) return g.K <= 3072;
     if (g.M <= 4 && g.K >= 4096) return false;
+    if (!waves_plan(g).one_round) return g.M > 8 ? g.K <= 1536 : g.K <= 1024 && cols * g.K <= 70'000'000;
     if (g.M <= 8 && g.K > 256 && g.K <= 512 && cols > 16384) return false;
-    if (!waves_plan(g).one_round) return g.M > 8 ? g.K <= 1024 : g.K <= (cols <= 65536 ? 768 : 256);
     return g.K <= 5120 && g.K <= 1536 + 128 * g.M + std::min<int64_t>(cols, 32768) / 32 + (g.ldb % 1024 ? 384 : 0);
 }
 

@@ -584,9 +584,9 @@ def test_kernel_choice_is_reported():
     assert name(M=1, N=4096, K=1792) == "mfma-i8-waves16x16x4" and name(M=1, N=4096, K=1808) == "mfma-i8-rows16-xcd"
     assert name(M=1, N=4112, K=2160) == "mfma-i8-waves16x32x4" and name(M=1, N=4112, K=2192) == "mfma-i8-rows16-xcd"
     assert name(M=1, N=28672, K=768) == "mfma-i8-waves16x128x4" and name(M=1, N=28672, K=512) == "mfma-i8-rows16-xcd"
-    assert name(M=1, N=40960, K=768) == "mfma-i8-waves16x64x1" and name(M=1, N=152064, K=1536) == "mfma-i8-rows16-xcd"
-    assert name(M=16, N=40960, K=1024) == "mfma-i8-waves16x64x1" and name(M=16, N=40960, K=1040) == "mfma-i8-rows16-xcd"
-    assert name(M=8, N=1024, K=2560) == "mfma-i8-waves16x16x4" and name(M=8, N=1024, K=2576) == "mfma-i8-rows16-tiles"
+    assert name(M=1, N=40960, K=1024) == "mfma-i8-waves16x64x1" and name(M=1, N=152064, K=512) == "mfma-i8-rows16-xcd"
+    assert name(M=16, N=40960, K=1536) == "mfma-i8-waves16x64x1" and name(M=16, N=40960, K=1552) == "mfma-i8-rows16-xcd"
+    assert name(M=8, N=1024, K=3072) == "mfma-i8-waves16x16x4" and name(M=8, N=1024, K=3088) == "mfma-i8-rows16-tiles"
     # A K of 80 steps and more over more tiles than it can be sliced for goes back to the split 128 tile.
     assert name(M=150, N=1408, K=5120) == "mfma-i8-direct128x128x64-splitk"
     assert name(M=128, N=1024, K=8192) == "mfma-i8-waves32x64x4-splitk"
